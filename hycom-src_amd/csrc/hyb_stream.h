@@ -923,6 +923,21 @@ struct FieldSink {  // T, S, tracers; th3d from T and S (hybgen.F90:1549-1569)
 #endif
     *a = x;
   }
+  // outputs kc..KN all take v (clamped); k is uniform over the wave, so a
+  // level is written as one row
+  HYB_HD void tail(int kc, int KN, const double* v, uint64_t) {
+    double th = 0.0;
+    if constexpr (NF >= 2)
+      if (th3d) th = sig(v[0], v[1]) - thbase;
+    for (int k = 1; k <= KN; k++) {
+      if (k < kc) continue;
+#pragma unroll
+      for (int f = 0; f < NF; f++)
+        if (f < nf) put(fp[f] + (int64_t)(k - 1) * S, v[f]);
+      if constexpr (NF >= 2)
+        if (th3d) put(th3d + (int64_t)(k - 1) * S, th);
+    }
+  }
   // clamp to [smin, smax] the outputs outside [lo, hi] (lo = smin and
   // hi = smax except in the mixed form, see walk_core)
   HYB_HD void fixup(const double* lo, const double* hi, const double* smin,
@@ -953,7 +968,7 @@ struct UvSink {  // u or v with the thin-layer rule (hybgen.F90:1858-1865)
   int64_t S;
   double ub;    // ubavg or vbavg at time level nl
   double ptop;  // prsf(kk+1)
-  const PO* po;
+  PO* po;
   uint64_t fix = 0;
   // With PoRecompute, the new dpu of layer kc (dpudpv.F90:92-103) is
   // written as output kc is: the walk asks for prsf(kc+1) just before it
@@ -970,6 +985,14 @@ struct UvSink {  // u or v with the thin-layer rule (hybgen.F90:1858-1865)
       uu[(int64_t)(kc - 1) * S] = -ub;
     }
     if constexpr (is_recompute<PO>::value) dpn[(int64_t)(kc - 1) * S] = po->dl;
+  }
+  // outputs kc..KN all take v (clamped), by the rule of emit
+  HYB_HD void tail(int kc, int KN, const double* v, uint64_t thick) {
+    for (int k = 1; k <= KN; k++) {
+      if (k < kc) continue;
+      (void)(*po)(k + 1);
+      emit(k, v, true, (thick >> (k - 1)) & 1ull);
+    }
   }
   HYB_HD void fixup(const double* lo, const double* hi, const double* smin,
                     const double* smax) {
@@ -1232,6 +1255,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
   // divisor is in [thin, 2^63] and every thickness or depth difference is 0
   // or in [2^-112, 2^61]
   constexpr bool FD64 = FDIV && !FAST;
+  (void)FD64;
   auto lcmb = [&](int l) -> bool { return (lcm >> (l - 1)) & 1ull; };
 
   // per-field state
@@ -1268,13 +1292,36 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
   auto load = [&](int f, int x) -> double {
     return fold(f, x, (x <= kp) ? static_cast<double>(fp[f][(int64_t)(x - 1) * S]) : 0.0);
   };
-  // the stored value of level min(x, kp), loaded without a use: with
-  // PD > 0 it is folded PD layer iterations later, so the load has that
-  // long to arrive (its value is discarded below kp)
-  auto raw = [&](int f, int x) -> RawT {
-    const int xc = x < kp ? x : kp;
-    return fp[f][(int64_t)(xc - 1) * S];
-  };
+  // The first window: every load is issued before any is used (levels
+  // clamped into the column; a value below kp or the bottom is not used).
+  auto lx = [&](int x) -> int { return x < K ? x : K; };
+  RawT r1[NF], r2[NF], r3[NF];
+#pragma unroll
+  for (int f = 0; f < NF; f++) {
+    if (f < nf) {
+      r1[f] = fp[f][0];
+      r2[f] = fp[f][(int64_t)(lx(2) - 1) * S];
+      r3[f] = fp[f][(int64_t)(lx(3) - 1) * S];
+#pragma unroll
+      for (int q = 0; q < PD; q++) sq[f][q] = fp[f][(int64_t)(lx(4 + q) - 1) * S];
+    }
+  }
+  const double pr1 = pi.raw(1), pr2 = pi.raw(lx(2)), pr3 = pi.raw(lx(3));
+#pragma unroll
+  for (int q = 0; q < PD; q++) prq[q] = pi.raw(lx(4 + q));
+  if constexpr (RAWT) {
+    tv1 = pi.thk(1);
+    tv2 = pi.thk(lx(2));
+    tv3 = pi.thk(lx(3));
+#pragma unroll
+    for (int q = 0; q < PQ; q++) tq[q] = pi.thk(lx(4 + q));
+  }
+  xl = 4 + PD;
+  // interfaces pi(l-1..l+3) at l = 1
+  double pv0 = 0.0, pv1 = pi.first(), pv2 = 0.0, pv3 = 0.0, pv4 = 0.0;
+  pv2 = pi.comb(pv1, pr1);
+  if (K >= 2) pv3 = pi.comb(pv2, pr2);
+  if (K >= 3) pv4 = pi.comb(pv3, pr3);
 #pragma unroll
   for (int f = 0; f < NF; f++) {
     s0[f] = s1[f] = s2[f] = s3[f] = 0.0;
@@ -1283,12 +1330,10 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     cst.asc[f] = cst.alc[f] = 0.0;
     cst.wc1[f] = cst.wc2[f] = cst.wz1[f] = cst.wz2[f] = cst.zw3l[f] = 0.0;
     if (f < nf) {
-      s1[f] = load(f, 1);
-      if (K >= 2) s2[f] = load(f, 2);
-      if (K >= 3) s3[f] = load(f, 3);
+      s1[f] = fold(f, 1, static_cast<double>(r1[f]));
+      if (K >= 2) s2[f] = fold(f, 2, static_cast<double>(r2[f]));
+      if (K >= 3) s3[f] = fold(f, 3, static_cast<double>(r3[f]));
       sfirst[f] = s1[f];
-#pragma unroll
-      for (int q = 0; q < PD; q++) sq[f][q] = (4 + q <= K) ? raw(f, 4 + q) : RawT{};
       if (METHOD == 2) cst.alc[f] = (CR)s1[f];  // al(1) = s(1)
       if (METHOD == 3) {                        // first sweep of layer 1
         cst.wc1[f] = (CR)s1[f];
@@ -1296,21 +1341,6 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
       }
     }
   }
-  // interfaces pi(l-1..l+3) at l = 1
-  double pv0 = 0.0, pv1 = pi.first(), pv2 = 0.0, pv3 = 0.0, pv4 = 0.0;
-  if (K + 1 >= 2) pv2 = pi.nextfrom(1, pv1);
-  if (K + 1 >= 3) pv3 = pi.nextfrom(2, pv2);
-  if (K + 1 >= 4) pv4 = pi.nextfrom(3, pv3);
-#pragma unroll
-  for (int q = 0; q < PD; q++) prq[q] = (4 + q <= K) ? pi.raw(4 + q) : 0.0;
-  if constexpr (RAWT) {
-    tv1 = pi.thk(1);
-    if (K >= 2) tv2 = pi.thk(2);
-    if (K >= 3) tv3 = pi.thk(3);
-#pragma unroll
-    for (int q = 0; q < PQ; q++) tq[q] = (4 + q <= K) ? pi.thk(4 + q) : 0.0;
-  }
-  xl = 4 + PD;
   // layers thicker than thin, known up to l+2 (the u/v store rule)
   uint64_t thick = 0;
   if (dmax(pv2 - pv1, thin) > thin) thick |= 1ull;
@@ -1335,12 +1365,11 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
   const double zb0 = dmax(po(1), pv1);
   int lt_c = 1;
   {
-    double pc = pv1;
-    while (lt_c < K) {
-      const double pn = pi.nextfrom(lt_c, pc);
-      if (!(pn < zb0)) break;
+    double pc = pv1, pn = pv2;  // pi(lt_c), pi(lt_c+1)
+    while (lt_c < K && pn < zb0) {
       lt_c++;
       pc = pn;
+      if (lt_c < K) pn = pi.nextfrom(lt_c, pc);
     }
   }
   double zt_c = zb0;
@@ -1359,14 +1388,15 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
   };
   // fold the levels below the window of layer l that are not folded yet:
   // those loaded ahead, then the rest (idempotent)
-  auto fold_rest = [&](int l) {
+  auto fold_rest = [&](int l, auto BI) {
+    constexpr int B = decltype(BI)::value;
 #pragma unroll
     for (int q = 0; q < PD; q++) {  // levels loaded ahead, not folded yet
       const int x = l + 3 + q;
       if (x <= K && x < xl) {
 #pragma unroll
         for (int f = 0; f < NF; f++)
-          if (f < nf) (void)fold(f, x, sq[f][q]);
+          if (f < nf) (void)fold(f, x, sq[f][(B + q) % PQ]);
       }
     }
     for (int x = xl; x <= K; x++) {
@@ -1389,8 +1419,15 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     kc = kc + 1;
   };
 
-#pragma unroll 1
-  for (int l = 1; l <= K; l++) {
+  // One layer.  BI is the slot, (l-1) mod PQ, of the look-ahead buffers that
+  // holds level l+3; the loop below runs PQ layers per turn so that each
+  // slot is a fixed set of registers.  (With slots that shift instead, every
+  // turn copies a register whose load has just been issued, and the copy
+  // waits for that load: the whole memory latency stood in every layer.)
+  // Returns false once every output is out.
+  auto layer = [&](int l, auto BI) __attribute__((always_inline)) -> bool {
+    constexpr int B = decltype(BI)::value;
+    constexpr bool FD64 = FDIV && !FAST;
     const double dprs_m = RAWT ? tv0 : pv1 - pv0, dprs_0 = RAWT ? tv1 : pv2 - pv1,
                  dprs_p = RAWT ? tv2 : pv3 - pv2, dprs_p2 = RAWT ? tv3 : pv4 - pv3;
     const double dpi_m = dmax(dprs_m, thin), dpi_0 = dmax(dprs_0, thin),
@@ -1462,14 +1499,17 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     // Every output still to come ends in this layer when it reaches the
     // bottom, and the walk stops here: fold the levels not read yet into
     // the column range now, before any of them is overwritten.
-    if (l < K && pil1 >= zx) fold_rest(l);
+    if (l < K && pil1 >= zx) fold_rest(l, BI);
     // ------------------------------------------ output in progress
     if (accon) {
       if (lb_act == l) {
         double v[NF];
         if (acc_thin) {
 #pragma unroll
-          for (int f = 0; f < NF; f++) v[f] = (kc != 1) ? prev[f] : sfirst[f];
+          for (int f = 0; f < NF; f++) {
+            const double a = prev[f], b = sfirst[f];
+            v[f] = (kc != 1) ? a : b;
+          }
         } else {
           const double xb = xof(zb_act);
           const double dpb = zb_act - pil;
@@ -1530,7 +1570,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     }
     // ------------------------------------------ outputs starting in layer l
     if (!accon && lt_c == l) {
-      while (kc <= KN) {
+      while (kc <= KN && !(zt_c >= zx)) {
         const double zt = zt_c;
         const double zb = dmin(po(kc + 1), zx);
         const bool ends_here = (l == K) || (pil1 >= zb);
@@ -1539,7 +1579,10 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
           double v[NF];
           if (thn) {
 #pragma unroll
-            for (int f = 0; f < NF; f++) v[f] = (kc != 1) ? prev[f] : sfirst[f];
+            for (int f = 0; f < NF; f++) {
+              const double a = prev[f], b = sfirst[f];
+              v[f] = (kc != 1) ? a : b;
+            }
           } else if (METHOD == 0) {
 #pragma unroll
             for (int f = 0; f < NF; f++) v[f] = s1[f];
@@ -1628,12 +1671,10 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
             for (int f = 0; f < NF; f++) {
               if (f < nf) {
                 // o = s(mid), with the fill; levels > l+2 are not written yet
-                double o;
-                if (mid == l) o = s1[f];
-                else if (mid == l + 1) o = s2[f];
-                else if (mid == l + 2) o = s3[f];
-                else if (kp <= l + 2) o = skp[f];
-                else o = static_cast<double>(fp[f][(int64_t)((mid < kp ? mid : kp) - 1) * S]);
+                const double w1 = s1[f], w2 = s2[f], w3 = s3[f], wk = skp[f];
+                double o = mid == l ? w1 : (mid == l + 1 ? w2 : (mid == l + 2 ? w3 : wk));
+                if (mid > l + 2 && kp > l + 2)
+                  o = static_cast<double>(fp[f][(int64_t)((mid < kp ? mid : kp) - 1) * S]);
                 ov[f] = o;
                 accc[f] = 0.0;
                 if (METHOD == 0) {
@@ -1653,11 +1694,16 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
         }
       }
     }
-    if (kc > KN) {
+    // The outputs below the bottom (zt >= zx) all take the last value; they
+    // are written after the loop, where every lane of the wave has reached
+    // its own bottom.  Written here, each lane's would run alone in the
+    // layer of its bottom: in waves over sloping ground about 110 turns of
+    // the loop above beside 36 layers (600x400x41 tile).
+    if (kc > KN || (!accon && zt_c >= zx)) {
       // every output is out; with fewer new layers than old ones the
       // levels below may not be read yet, and the range covers them all
-      if (KO > 0) fold_rest(l);
-      break;
+      if (KO > 0) fold_rest(l, BI);
+      return false;
     }
     // ------------------------------------------ slide to layer l+1
     // The slide's look-ahead loads issue at raised wave priority, ahead of
@@ -1673,20 +1719,14 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     if (PD == 0) {
       pv4 = (l + 4 <= K + 1) ? pi.nextfrom(l + 3, top) : 0.0;
     } else {
-      pv4 = (l + 4 <= K + 1) ? pi.comb(top, prq[0]) : 0.0;
-#pragma unroll
-      for (int q = 0; q < PD - 1; q++) prq[q] = prq[q + 1];
-      prq[PQ - 1] = (l + 3 + PD <= K) ? pi.raw(l + 3 + PD) : 0.0;
+      pv4 = (l + 4 <= K + 1) ? pi.comb(top, prq[B]) : 0.0;
     }
     if (l + 3 <= K && dmax(pv4 - pv3, thin) > thin) thick |= 1ull << (l + 2);
     if constexpr (RAWT) {
       tv0 = tv1;
       tv1 = tv2;
       tv2 = tv3;
-      tv3 = (l + 3 <= K) ? tq[0] : 0.0;
-#pragma unroll
-      for (int q = 0; q < PQ - 1; q++) tq[q] = tq[q + 1];
-      tq[PQ - 1] = (l + 3 + PQ <= K) ? pi.thk(l + 3 + PQ) : 0.0;
+      tv3 = (l + 3 <= K) ? tq[B] : 0.0;
     }
 #pragma unroll
     for (int f = 0; f < NF; f++) {
@@ -1696,22 +1736,60 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
       if (PD == 0) {
         s3[f] = (f < nf && xl <= K) ? load(f, xl) : 0.0;
       } else {
-        s3[f] = (f < nf && l + 3 <= K) ? fold(f, l + 3, sq[f][0]) : 0.0;
+        s3[f] = (f < nf && l + 3 <= K) ? fold(f, l + 3, sq[f][B]) : 0.0;
+      }
+    }
+    // slot B is free: level l+3+PQ goes into it.  Clamped into the column
+    // and unconditional for the interfaces; the fields' levels below kp are
+    // not loaded (the fill takes their place).
+    if (PD > 0 || RAWT) {
+      const int xn = l + 3 + PQ;
+      const int xk = xn < K ? xn : K;
+      if (PD > 0) prq[B] = pi.raw(xk);
+      if constexpr (RAWT) tq[B] = pi.thk(xk);
+      if (PD > 0 && xn <= kp) {
 #pragma unroll
-        for (int q = 0; q < PD - 1; q++) sq[f][q] = sq[f][q + 1];
-        sq[f][PQ - 1] = (f < nf && xl <= K) ? raw(f, xl) : RawT{};
+        for (int f = 0; f < NF; f++)
+          if (f < nf) sq[f][B] = fp[f][(int64_t)(xn - 1) * S];
       }
     }
 #if defined(__HIP_DEVICE_COMPILE__)
     __builtin_amdgcn_s_setprio(0);
 #endif
     xl++;
+    return true;
+  };
+  {
+    int l = 1;
+#pragma unroll 1
+    for (;;) {
+      if (!layer(l, std::integral_constant<int, 0>{}) || ++l > K) break;
+      if constexpr (PQ > 1)
+        if (!layer(l, std::integral_constant<int, 1>{}) || ++l > K) break;
+      if constexpr (PQ > 2)
+        if (!layer(l, std::integral_constant<int, 2>{}) || ++l > K) break;
+      if constexpr (PQ > 3)
+        if (!layer(l, std::integral_constant<int, 3>{}) || ++l > K) break;
+    }
   }
   double lo[NF], hi[NF];
 #pragma unroll
   for (int f = 0; f < NF; f++) {
     lo[f] = FAST ? smin[f] - slack(f) : smin[f];
     hi[f] = FAST ? smax[f] + slack(f) : smax[f];
+  }
+  if (kc <= KN) {
+    // prev is the last output before its clamp; the range is complete now
+    double tl[NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      const double a = prev[f], b = sfirst[f];
+      double x = (kc != 1) ? a : b;
+      x = (x < lo[f]) ? smin[f] : x;
+      x = (x > hi[f]) ? smax[f] : x;
+      tl[f] = x;
+    }
+    sink.tail(kc, KN, tl, thick);
   }
   sink.fixup(lo, hi, smin, smax);
 }
