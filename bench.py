@@ -27,7 +27,7 @@ METRIC = "column-layers remapped/s, FP64 vs mixed, GLBb tile; p50/p99 request la
 HBM_PEAK_GBS = 8000.0
 PHASES = ["column", "halo", "uv", "ra", "halo2", "uv2", "regrid", "remap"]
 # kernel of each p-column remap variant (hycom_hybgen_tune knob 0)
-REMAP_KERNELS = {3: "k_remap_s<{m},3,2>"}
+REMAP_KERNELS = {3: "k_remap_s<{m},2,false>"}
 
 
 def bytes_per_column_phase_a(K, T):

@@ -30,7 +30,7 @@ int uv_method_of(const KParams& P);
 // remap_variant picks the p-column remap kernel (hyb_k_remap.inc),
 // uv_prefetch the prefetch depth of the u/v walk (0, 2 or 4).
 struct StreamTuning {
-  int remap_variant = 3;  // 3 fields per walk, 2 levels loaded ahead (fastest measured)
+  int remap_variant = 3;  // the only one built
   int uv_prefetch = 4;
   int uv_recompute = 1;  // u/v new thicknesses formed again from p, no LDS (fastest measured)
   int regrid_ahead = 1;  // the regrid's window loaded one iteration ahead (fastest measured)

@@ -844,6 +844,7 @@ struct PoRecomputeT {
   double prv = 0.0, cur = 0.0, b = 0.0;  // prsf(k-1), prsf(k), min(depthu, p-mean at k)
   double dl = 0.0;                       // the new thickness of layer k-1 (cur = prv + dl)
   double q0[A], q1[A];                   // p at levels k+1..k+A of both points, loaded ahead
+  int64_t at = 0;                        // offset of level k+A, clamped into the column
   int k = 0;                             // 0 until the first request
   HYB_HD PoRecomputeT(const double* a0, const double* a1, int64_t s, double du, int kk)
       : p0(a0), p1(a1), S(s), depthu(du), k1(kk + 1) {
@@ -859,9 +860,9 @@ struct PoRecomputeT {
       k = 1;
 #pragma unroll
       for (int q = 0; q < A; q++) {
-        const int x = 1 + q < k1 ? 1 + q : k1 - 1;
-        q0[q] = p0[(int64_t)x * S];
-        q1[q] = p1[(int64_t)x * S];
+        at = (int64_t)(1 + q < k1 ? 1 + q : k1 - 1) * S;
+        q0[q] = p0[at];
+        q1[q] = p1[at];
       }
     }
     while (k < kq) {
@@ -877,10 +878,9 @@ struct PoRecomputeT {
         q0[q] = q0[q + 1];
         q1[q] = q1[q + 1];
       }
-      // level k+A-1, clamped into the column (values beyond it unused)
-      const int x = k + A - 1 < k1 ? k + A - 1 : k1 - 1;
-      q0[A - 1] = p0[(int64_t)x * S];
-      q1[A - 1] = p1[(int64_t)x * S];
+      if (k + A - 1 < k1) at += S;
+      q0[A - 1] = p0[at];
+      q1[A - 1] = p1[at];
     }
     return cur;
   }
@@ -891,8 +891,8 @@ struct is_recompute : std::false_type {};
 template <int A>
 struct is_recompute<PoRecomputeT<A>> : std::true_type {};
 
-// Output sinks.  emit(kc, v, certain, thick): v[f] is output kc of field
-// f before the clamp; certain means it lies inside the range of the input
+// Output sinks.  emit(kc, at, v, certain, thick): v[f] is output kc of field
+// f before the clamp, at its offset (kc-1)*S from level 1; certain means it lies inside the range of the input
 // levels read so far, so the clamp against the whole column cannot change
 // it.  fixup() clamps the others once the column range is known.
 // NT: outputs written with non-temporal stores (streamed past the caches)
@@ -904,14 +904,14 @@ struct FieldSink {  // T, S, tracers; th3d from T and S (hybgen.F90:1549-1569)
   double thbase;
   int64_t S;
   uint64_t fix = 0;
-  HYB_HD void emit(int kc, const double* v, bool certain, bool) {
+  HYB_HD void emit(int kc, int64_t at, const double* v, bool certain, bool) {
 #pragma unroll
     for (int f = 0; f < NF; f++)
-      if (f < nf) put(fp[f] + (int64_t)(kc - 1) * S, v[f]);
+      if (f < nf) put(fp[f] + at, v[f]);
     if (!certain) {
       fix |= 1ull << (kc - 1);
     } else if constexpr (NF >= 2) {  // th3d needs T and S in the same walk
-      if (th3d) put(th3d + (int64_t)(kc - 1) * S, sig(v[0], v[1]) - thbase);
+      if (th3d) put(th3d + at, sig(v[0], v[1]) - thbase);
     }
   }
   HYB_HD static void put(double* a, double x) {
@@ -977,21 +977,21 @@ struct UvSink {  // u or v with the thin-layer rule (hybgen.F90:1858-1865)
   // two layers above their index (the in-place test of uv_stream), and the
   // old interfaces are summed PD+3 layers ahead of the walk.
   double* dpn = nullptr;
-  HYB_HD void emit(int kc, const double* v, bool certain, bool thick) {
+  HYB_HD void emit(int kc, int64_t at, const double* v, bool certain, bool thick) {
     if (thick || po->prv <= ptop - kOnemm) {
-      uu[(int64_t)(kc - 1) * S] = v[0];
+      uu[at] = v[0];
       if (!certain) fix |= 1ull << (kc - 1);
     } else {
-      uu[(int64_t)(kc - 1) * S] = -ub;
+      uu[at] = -ub;
     }
-    if constexpr (is_recompute<PO>::value) dpn[(int64_t)(kc - 1) * S] = po->dl;
+    if constexpr (is_recompute<PO>::value) dpn[at] = po->dl;
   }
   // outputs kc..KN all take v (clamped), by the rule of emit
   HYB_HD void tail(int kc, int KN, const double* v, uint64_t thick) {
     for (int k = 1; k <= KN; k++) {
       if (k < kc) continue;
       (void)(*po)(k + 1);
-      emit(k, v, true, (thick >> (k - 1)) & 1ull);
+      emit(k, (int64_t)(k - 1) * S, v, true, (thick >> (k - 1)) & 1ull);
     }
   }
   HYB_HD void fixup(const double* lo, const double* hi, const double* smin,
@@ -1020,6 +1020,41 @@ struct CoefState {
   R zw3l[NF];                             // WENO interface value zw3(l)
   R qdpjp_l, wq_l;                        // PPM qdpjp(l); WENO 1/(dp(l)+dp(l+1))
 };
+
+// x in a register of its own: a look-ahead value leaves its slot by this
+// move, so the slot is free for the next load (without it the allocator
+// keeps x in the slot, loads the next value elsewhere, and copies it back
+// at the end of the turn, waiting for the load there).
+HYB_HD double leave_slot(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y;
+  asm("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
+  return y;
+#else
+  return x;
+#endif
+}
+
+// sign(min(|a|,|b|,|c|), b) for finite or infinite a, b, c, in three
+// instructions on the device (NaN operands do not reach a use of it: the
+// callers take it only where a product of the differences is positive)
+HYB_HD double min3_sign(double a, double b, double c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double m;
+  asm("v_min_f64 %0, |%1|, |%2|" : "=v"(m) : "v"(a), "v"(b));
+  asm("v_min_f64 %0, %1, |%2|" : "=v"(m) : "v"(m), "v"(c));
+  return __builtin_copysign(m, b);
+#else
+  const double x = fabs(a), y = fabs(b), z = fabs(c);
+  const double m = x < y ? x : y;
+  return copysign(m < z ? m : z, b);
+#endif
+}
+HYB_HD float min3_sign(float a, float b, float c) {
+  const float x = fabsf(a), y = fabsf(b), z = fabsf(c);
+  const float m = x < y ? x : y;
+  return copysignf(m < z ? m : z, b);
+}
 
 template <class R>
 HYB_HD R gmax(R a, R b) { return a > b ? a : b; }
@@ -1108,7 +1143,7 @@ __attribute__((always_inline)) HYB_HD void coef_layer(
           const R slj = s2[f] - s1[f];
           const R srj = s3[f] - s2[f];
           const R scj = dpq3 * (dp2jp_l * srj * qdpjp_n + dpj2p_n * slj * st.qdpjp_l);
-          const R asv = gsign(gmin3(gabs(R(2) * slj), gabs(scj), gabs(R(2) * srj)), scj);
+          const R asv = min3_sign(R(2) * slj, scj, R(2) * srj);
           as_n = (do_as && slj * srj > R(0)) ? asv : R(0);
         }
         if (jn == K) {
@@ -1374,6 +1409,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
   }
   double zt_c = zb0;
   int kc = 1;
+  int64_t kat = 0;  // (kc-1)*S
   bool accon = false, acc_thin = false;
   int lb_act = 0;
   double zt_act = 0.0, zb_act = 0.0;
@@ -1415,8 +1451,9 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
         prev[f] = v[f];
         if (!(v[f] >= smin[f] && v[f] <= smax[f])) certain = false;
       }
-    sink.emit(kc, v, certain, (thick >> (kc - 1)) & 1ull);
+    sink.emit(kc, kat, v, certain, (thick >> (kc - 1)) & 1ull);
     kc = kc + 1;
+    kat = kat + S;
   };
 
   // One layer.  BI is the slot, (l-1) mod PQ, of the look-ahead buffers that
@@ -1671,10 +1708,13 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
             for (int f = 0; f < NF; f++) {
               if (f < nf) {
                 // o = s(mid), with the fill; levels > l+2 are not written yet
-                const double w1 = s1[f], w2 = s2[f], w3 = s3[f], wk = skp[f];
-                double o = mid == l ? w1 : (mid == l + 1 ? w2 : (mid == l + 2 ? w3 : wk));
-                if (mid > l + 2 && kp > l + 2)
-                  o = static_cast<double>(fp[f][(int64_t)((mid < kp ? mid : kp) - 1) * S]);
+                double o = s1[f];
+                if (mid != l) {
+                  const double w2 = s2[f], w3 = s3[f], wk = skp[f];
+                  o = mid == l + 1 ? w2 : (mid == l + 2 ? w3 : wk);
+                  if (mid > l + 2 && kp > l + 2)
+                    o = static_cast<double>(fp[f][(int64_t)((mid < kp ? mid : kp) - 1) * S]);
+                }
                 ov[f] = o;
                 accc[f] = 0.0;
                 if (METHOD == 0) {
@@ -1719,7 +1759,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     if (PD == 0) {
       pv4 = (l + 4 <= K + 1) ? pi.nextfrom(l + 3, top) : 0.0;
     } else {
-      pv4 = (l + 4 <= K + 1) ? pi.comb(top, prq[B]) : 0.0;
+      pv4 = (l + 4 <= K + 1) ? pi.comb(top, leave_slot(prq[B])) : 0.0;
     }
     if (l + 3 <= K && dmax(pv4 - pv3, thin) > thin) thick |= 1ull << (l + 2);
     if constexpr (RAWT) {
@@ -1944,6 +1984,49 @@ HYB_HDI SplitInterfaces stage_split(double* row, int ld, const double* pg, int64
   stage_column(row, ld, pg + S, S, n);
   SplitInterfaces po{row, pg, S, ld, K + 1, n + 1, top, bot};
   return po;
+}
+
+// The part of stage_interfaces that wave w of nw does: every nw-th level,
+// 8 loads in flight before the first is stored.
+HYB_HDI StagedInterfaces stage_interfaces_part(double* row, int ld, const double* pg, int64_t S,
+                                               int K, int w, int nw) {
+  const double top = pg[0], bot = pg[(int64_t)K * S];
+  for (int k0 = w; k0 < K - 1; k0 += 8 * nw) {
+    double t[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int k = k0 + q * nw;
+      t[q] = pg[(int64_t)(k < K - 1 ? k + 1 : K) * S];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (k0 + q * nw < K - 1) row[(int64_t)(k0 + q * nw) * ld] = t[q];
+  }
+  return StagedInterfaces{row, ld, K + 1, top, bot};
+}
+
+// Waves of a remap block: one per pair of fields, at most four; more pairs
+// take more blocks.
+constexpr int kRemapWaves = 4;
+HYB_HD int field_pairs(const KParams& P) { return (2 + P.ntracr + 1) / 2; }
+HYB_HD int remap_waves(int pairs) { return pairs < kRemapWaves ? pairs : kRemapWaves; }
+HYB_HD int remap_blocks(int pairs) { return (pairs + kRemapWaves - 1) / kRemapWaves; }
+
+// The remap of pair q of a column's fields: fields 2q and 2q+1 (field 0 is
+// T, 1 is S, 2.. the tracers), or the last one alone.
+template <int METHOD, int PD, bool FAST, class PO>
+HYB_HDI void remap_pair(const KParams& P, const View& V, const Scratch& W, int64_t c0, int n,
+                        int kpw, int q, PO& po) {
+  const int K = P.kk;
+  const int kp = kpw & 0xffff;
+  const uint64_t lcm = W.lcm[c0];
+  const double* pres = W.pres + c0;
+  const double zx = pres[(int64_t)K * V.NIJ];
+  const int g0 = 2 * q, r = 2 + P.ntracr - g0;
+  if (r >= 2)
+    remap_walk<METHOD, 2, PD, FAST, false>(P, V, c0, n, g0, K, zx, pres, kp, lcm, po);
+  else if (r == 1)
+    remap_walk<METHOD, 1, PD, FAST, false>(P, V, c0, n, g0, K, zx, pres, kp, lcm, po);
 }
 
 // the last RA walk, over r < NF fields (r = 0: none)

@@ -240,8 +240,8 @@ int hycom_hybgen_set_kernel_path(int path);
 
 /* Variants of the streaming kernels (measurement and tuning; no reference
  * counterpart; results are bitwise the same for every value).  knob 0:
- * p-column remap variant, only 3 is built (3 fields per walk, 2 levels
- * loaded ahead, new interfaces staged in LDS); knob 1: levels loaded ahead
+ * p-column remap variant, only 3 is built (a wave per pair of fields, 2
+ * levels loaded ahead, new interfaces staged in LDS); knob 1: levels loaded ahead
  * by the u/v walk, 0, 2 or 4 (the default); knob 2: the u/v walk's new
  * thicknesses kept in LDS (0) or formed again from p as the walk needs them
  * (1, the default, no LDS); knob 3: the regrid's window loaded one
