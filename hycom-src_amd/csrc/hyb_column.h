@@ -1073,6 +1073,28 @@ HYB_HD void p_halo_icol(const KParams& P, const View& V, int j, int k) {
   }
 }
 
+// The same halo in one pass, every value taken from the interior: t in
+// [0, ii) the two points of column t+1's j-rows, then rows 0..jj+1 of the
+// i-columns (their corners are halo-row values: vland, or the row the halo row
+// copies).
+HYB_HD void p_halo_point(const KParams& P, const View& V, int t, int k) {
+  if (t < P.ii) {
+    p_halo_jrow(P, V, t + 1, k);
+    return;
+  }
+  double* p = V.p + lev(V, k);
+  const int j = t - P.ii;
+  const bool edge = j == 0 || j == P.jj + 1;
+  double w = P.vland, e = P.vland;
+  if (!(P.nreg == 0 || P.nreg == 4) && !(edge && P.nreg <= 2)) {
+    const int js = j == 0 ? P.jj : (j == P.jj + 1 ? 1 : j);
+    w = p[ij_of(V, P.ii, js)];
+    e = p[ij_of(V, 1, js)];
+  }
+  p[ij_of(V, 0, j)] = w;
+  p[ij_of(V, P.ii + 1, j)] = e;
+}
+
 // Scratch shared by the streaming column kernels.  pres level k of column
 // c0 is pres[c0 + (k-1)*NIJ]; the record words are indexed by c0.
 struct Scratch {

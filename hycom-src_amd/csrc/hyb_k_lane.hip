@@ -45,14 +45,23 @@ __global__ void __launch_bounds__(kBlock) k_phase_c(KParams P, View V, int nl) {
   point_c<KC>(P, V, i, j, nl, isv);
 }
 
-__global__ void __launch_bounds__(kWave) k_remap_fb(KParams P, View V, Scratch W, int n) {
+// the columns and the u- and v-points left over, in one launch (z: p, u, v)
+template <int KC>
+__global__ void __launch_bounds__(kWave) k_fb(KParams P, View V, Scratch W, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
   int j = blockIdx.y + 1;
   if (i > P.ii) return;
   const int64_t c0 = ij_of(V, i, j);
-  if (V.ip[c0] == 0) return;
-  if (!(W.kp[c0] & kUnsafe)) return;
-  remap_fallback(P, V, W, i, j, n);
+  if (blockIdx.z == 0) {
+    if (V.ip[c0] == 0) return;
+    if (!(W.kp[c0] & kUnsafe)) return;
+    remap_fallback(P, V, W, i, j, n);
+  } else {
+    const bool isv = blockIdx.z == 2;
+    if ((isv ? V.iv : V.iu)[c0] == 0) return;
+    if (W.uvf[c0 + (isv ? V.NIJ : 0)] == 0) return;
+    point_c<KC>(P, V, i, j, n, isv);
+  }
 }
 
 template <int KC>
@@ -106,16 +115,15 @@ void launch_ra_lane(const KParams& P, const View& V, int m, int n, hipStream_t s
   HYB_KC_DISPATCH(P.kk, hipLaunchKernelGGL(k_phase_ra<KC>, g2, dim3(kBlock), 0, s, P, V, m, n));
 }
 
-void launch_remap_fallback(const KParams& P, const View& V, const Scratch& W, int n,
-                           hipStream_t s) {
-  dim3 gw2((P.ii + kWave - 1) / kWave, P.jj);
-  hipLaunchKernelGGL(k_remap_fb, gw2, dim3(kWave), 0, s, P, V, W, n);
-}
-
 void launch_ra_fallback(const KParams& P, const View& V, const Scratch& W, int m, int n,
                         hipStream_t s) {
   dim3 gw2((P.ii + kWave - 1) / kWave, P.jj);
   HYB_KC_DISPATCH(P.kk, hipLaunchKernelGGL(k_ra_fb<KC>, gw2, dim3(kWave), 0, s, P, V, W, m, n));
+}
+
+void launch_fallbacks(const KParams& P, const View& V, const Scratch& W, int n, hipStream_t s) {
+  dim3 g((P.ii + kWave - 1) / kWave, P.jj, 3);
+  HYB_KC_DISPATCH(P.kk, hipLaunchKernelGGL(k_fb<KC>, g, dim3(kWave), 0, s, P, V, W, n));
 }
 
 void launch_uv_fallback(const KParams& P, const View& V, const Scratch& W, int nl,

@@ -7,19 +7,11 @@
 
 namespace hyb {
 
-// p halo, levels 2..kk+1: first the j rows (mod_xc_sm.h:1374-1392), then
-// the i columns including the corners (1394-1424).
-__global__ void k_halo_j(KParams P, View V) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  int k = blockIdx.y + 2;
-  if (i > P.ii) return;
-  p_halo_jrow(P, V, i, k);
-}
-__global__ void k_halo_i(KParams P, View V) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;  // 0..jj+1
-  int k = blockIdx.y + 2;
-  if (j > P.jj + 1) return;
-  p_halo_icol(P, V, j, k);
+// p halo, levels 2..kk+1: the j rows and the i columns with the corners
+// (mod_xc_sm.h:1374-1424) in one launch.
+__global__ void k_halo(KParams P, View V) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < P.ii + P.jj + 2) p_halo_point(P, V, t, blockIdx.y + 2);
 }
 
 // diagnostic tracers itracr(801..803): copy before (hybgen.F90:44-87),
@@ -112,10 +104,8 @@ hipError_t launch_scan_finite(const KParams& P, const View& V, int n, int32_t* o
 }
 
 hipError_t launch_halo(const KParams& P, const View& V, hipStream_t s) {
-  dim3 gj((P.ii + kBlock - 1) / kBlock, P.kk);
-  hipLaunchKernelGGL(k_halo_j, gj, dim3(kBlock), 0, s, P, V);
-  dim3 gi((P.jj + 2 + kBlock - 1) / kBlock, P.kk);
-  hipLaunchKernelGGL(k_halo_i, gi, dim3(kBlock), 0, s, P, V);
+  dim3 g((P.ii + P.jj + 2 + kBlock - 1) / kBlock, P.kk);
+  hipLaunchKernelGGL(k_halo, g, dim3(kBlock), 0, s, P, V);
   return hipGetLastError();
 }
 

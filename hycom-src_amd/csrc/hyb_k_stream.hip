@@ -60,6 +60,20 @@ bool stream_path_ok(const KParams& P) { return P.nhybrd == P.kk; }
 
 int uv_method_of(const KParams& P) { return uv_method(P); }
 
+// The remap and the u/v phase in one launch, where a launch of either leaves
+// much of the chip idle: the remap takes a wave per 64 columns and pair of
+// fields, u/v two waves per 64 columns, and the chip holds 3072 of the
+// combined kernel's waves.  Up to eight times that, one launch against two:
+// 40x30x16 91 against 129 us, 150x100x32 202 against 279 us, 331x277x22 327
+// against 352 us, 600x400x41 (20 000 waves) 1084 against 1147 us.  Beyond, the
+// two kernels' streams through memory get in each other's way: 1500x1000x41
+// WENO (96 000 waves) 5.2 against 4.2 ms.
+static bool one_launch(const KParams& P, const StreamTuning& tune) {
+  const int64_t tiles = (int64_t)((P.ii + kAlignPad + kWave - 1) / kWave) * P.jj;
+  return tune.uv_recompute && tune.uv_prefetch == 4 && !tune.concurrent_uv &&
+         tiles * (field_pairs(P) + 2) <= 8 * 3072;
+}
+
 hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& W, int m,
                                 int n, int raflag, const StreamTuning& tune, hipStream_t s,
                                 PhaseTimer* T) {
@@ -71,6 +85,8 @@ hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& 
   std::unique_lock<std::mutex> fork_lock(g_fork_mu, std::defer_lock);
   Fork* F = nullptr;
   hipStream_t su = s;  // stream of the u/v phase
+  bool uv_done = false;
+  hipError_t e = hipSuccess;
   {
     PhaseMark pm(T, s, 0);
     {
@@ -80,21 +96,28 @@ hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& 
       else
         hipLaunchKernelGGL(k_regrid_s, g2, blk, 0, s, P, V, W, n);
     }
-    if (tune.concurrent_uv) {
-      hipError_t e = fork_of(&F);
-      if (e != hipSuccess) return e;
-      fork_lock.lock();
-      if ((e = hipEventRecord(F->fork, s)) != hipSuccess) return e;
-      if ((e = hipStreamWaitEvent(F->s2, F->fork, 0)) != hipSuccess) return e;
-      su = F->s2;
-      {
-        PhaseMark pu(T, su, 1);
-        if ((e = launch_halo(P, V, su)) != hipSuccess) return e;
-      }
-      PhaseMark pu(T, su, 2);
-      launch_uv_stream(P, V, W, n, tune, su);
-    }
     {
+      PhaseMark ph(T, s, 1);
+      if ((e = launch_halo(P, V, s)) != hipSuccess) return e;
+    }
+    if (!T && one_launch(P, tune)) {
+      switch (P.hybmap) {
+        case 0: launch_remap_uv_m0(P, V, W, n, s); break;
+        case 1: launch_remap_uv_m1(P, V, W, n, s); break;
+        case 2: launch_remap_uv_m2(P, V, W, n, s); break;
+        default: launch_remap_uv_m3(P, V, W, n, s); break;
+      }
+      uv_done = true;
+    } else {
+      if (tune.concurrent_uv) {
+        if ((e = fork_of(&F)) != hipSuccess) return e;
+        fork_lock.lock();
+        if ((e = hipEventRecord(F->fork, s)) != hipSuccess) return e;
+        if ((e = hipStreamWaitEvent(F->s2, F->fork, 0)) != hipSuccess) return e;
+        su = F->s2;
+        PhaseMark pu(T, su, 2);
+        launch_uv_stream(P, V, W, n, tune, su);
+      }
       PhaseMark pk(T, s, 7);
       const int rv = tune.remap_variant;
       switch (P.hybmap) {
@@ -104,23 +127,18 @@ hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& 
         default: launch_remap_stream_m3(P, V, W, n, rv, s); break;
       }
     }
-    launch_remap_fallback(P, V, W, n, s);
   }
-  launch_diag_post(P, V, n, s);
-  hipError_t e;
   if (F) {  // join: the caller's stream waits for the u/v phase
     if ((e = hipEventRecord(F->join, su)) != hipSuccess) return e;
     if ((e = hipStreamWaitEvent(s, F->join, 0)) != hipSuccess) return e;
     fork_lock.unlock();
+    launch_fallbacks(P, V, W, n, s);
   } else {
-    {
-      PhaseMark pm(T, s, 1);
-      e = launch_halo(P, V, s);
-    }
-    if (e != hipSuccess) return e;
     PhaseMark pm(T, s, 2);
-    launch_uv_stream(P, V, W, n, tune, s);
+    if (!uv_done) launch_uv_stream(P, V, W, n, tune, s);
+    launch_fallbacks(P, V, W, n, s);
   }
+  launch_diag_post(P, V, n, s);
   if (raflag) {
     {
       PhaseMark pm(T, s, 3);
@@ -139,6 +157,7 @@ hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& 
     if (e != hipSuccess) return e;
     PhaseMark pm(T, s, 5);
     launch_uv_stream(P, V, W, m, tune, s);
+    launch_uv_fallback(P, V, W, m, s);
   }
   return hipGetLastError();
 }

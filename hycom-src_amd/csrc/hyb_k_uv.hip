@@ -7,6 +7,13 @@
 
 namespace hyb {
 
+// A wave per 64 u- or v-points.  Bound by the latency of its walk's loads at
+// the occupancy its registers allow: with the column's arrays addressed from
+// uniform bases the walk takes 125 VGPRs, 4 waves a SIMD (138 and 3 with a
+// pointer per lane and array), and every word of a layer is asked for one
+// layer ahead and waited for in one place (PoRecompute).  One slot per array
+// (PD = 1) beats two (133 VGPRs, 3 waves): 2250x1649x41 call 10.4 against
+// 11.0 ms, 1500x1000x41 WENO 4.03 against 4.29 ms; before, 10.8 and 4.2 ms.
 template <int METHOD, int PD, bool MIXED = false, bool RECOMP = false>
 __global__ void __launch_bounds__(kWave) k_uv_s(KParams P, View V, Scratch W, int nl) {
   extern __shared__ double lds[];
@@ -29,9 +36,9 @@ static void uv_stream_m(const KParams& P, const View& V, const Scratch& W, int n
   dim3 gw3((P.ii + kAlignPad + kWave - 1) / kWave, P.jj, 2);
   const size_t lds = RECOMP ? 0 : sizeof(double) * P.kk * kWave;
   if (P.precision == 1)
-    hipLaunchKernelGGL((k_uv_s<M, 4, true, RECOMP>), gw3, w1, lds, s, P, V, W, nl);
+    hipLaunchKernelGGL((k_uv_s<M, 1, true, RECOMP>), gw3, w1, lds, s, P, V, W, nl);
   else if (pd == 4)
-    hipLaunchKernelGGL((k_uv_s<M, 4, false, RECOMP>), gw3, w1, lds, s, P, V, W, nl);
+    hipLaunchKernelGGL((k_uv_s<M, 1, false, RECOMP>), gw3, w1, lds, s, P, V, W, nl);
   else if (pd > 0)
     hipLaunchKernelGGL((k_uv_s<M, 2, false, RECOMP>), gw3, w1, lds, s, P, V, W, nl);
   else
@@ -51,7 +58,6 @@ void launch_uv_stream(const KParams& P, const View& V, const Scratch& W, int nl,
     else if (m == 1) uv_stream_m<1, false>(P, V, W, nl, pd, s);
     else uv_stream_m<3, false>(P, V, W, nl, pd, s);
   }
-  launch_uv_fallback(P, V, W, nl, s);
 }
 
 }  // namespace hyb

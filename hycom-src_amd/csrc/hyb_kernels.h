@@ -28,7 +28,7 @@ bool stream_path_ok(const KParams& P);
 int uv_method_of(const KParams& P);
 // Kernel variants of the streaming family (measurement and tuning):
 // remap_variant picks the p-column remap kernel (hyb_k_remap.inc),
-// uv_prefetch the prefetch depth of the u/v walk (0, 2 or 4).
+// uv_prefetch the look-ahead of the u/v walk (0, 2 or 4).
 struct StreamTuning {
   int remap_variant = 3;  // the only one built
   int uv_prefetch = 4;

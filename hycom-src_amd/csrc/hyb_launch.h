@@ -29,8 +29,8 @@ struct PhaseMark {
   }
 };
 
-// hyb_k_uv.hip: the streaming u/v kernels of time level nl, then the
-// fallback points they flagged
+// hyb_k_uv.hip: the streaming u/v kernels of time level nl (the points they
+// flag are left to launch_uv_fallback or launch_fallbacks)
 void launch_uv_stream(const KParams& P, const View& V, const Scratch& W, int nl,
                       const StreamTuning& tune, hipStream_t s);
 // hyb_k_misc.hip
@@ -40,15 +40,15 @@ void launch_diag_post(const KParams& P, const View& V, int n, hipStream_t s);
 // hyb_k_lane.hip: per-lane-array kernels used by the other families too
 void launch_uv_lane(const KParams& P, const View& V, int nl, hipStream_t s);
 void launch_ra_lane(const KParams& P, const View& V, int m, int n, hipStream_t s);
-void launch_remap_fallback(const KParams& P, const View& V, const Scratch& W, int n,
-                           hipStream_t s);
+// both in one launch
+void launch_fallbacks(const KParams& P, const View& V, const Scratch& W, int n, hipStream_t s);
 void launch_uv_fallback(const KParams& P, const View& V, const Scratch& W, int nl,
                         hipStream_t s);
 // column_ra for the columns the streaming RA kernel flagged in W.kp
 void launch_ra_fallback(const KParams& P, const View& V, const Scratch& W, int m, int n,
                         hipStream_t s);
 // hyb_k_remap_m*.hip: streaming remap of the p-columns for one remapper;
-// variant selects fields per walk and the prefetch depth
+// variant 3, the only one built
 void launch_remap_stream_m0(const KParams& P, const View& V, const Scratch& W, int n,
                             int variant, hipStream_t s);
 void launch_remap_stream_m1(const KParams& P, const View& V, const Scratch& W, int n,
@@ -57,6 +57,12 @@ void launch_remap_stream_m2(const KParams& P, const View& V, const Scratch& W, i
                             int variant, hipStream_t s);
 void launch_remap_stream_m3(const KParams& P, const View& V, const Scratch& W, int n,
                             int variant, hipStream_t s);
+// the same remap with the u/v phase of time level n in one launch (after the
+// p halo)
+void launch_remap_uv_m0(const KParams& P, const View& V, const Scratch& W, int n, hipStream_t s);
+void launch_remap_uv_m1(const KParams& P, const View& V, const Scratch& W, int n, hipStream_t s);
+void launch_remap_uv_m2(const KParams& P, const View& V, const Scratch& W, int n, hipStream_t s);
+void launch_remap_uv_m3(const KParams& P, const View& V, const Scratch& W, int n, hipStream_t s);
 // the Robert-Asselin branch (hybgencj) on the streaming design, per remapper
 void launch_ra_stream_m0(const KParams& P, const View& V, const Scratch& W, int m, int n,
                          hipStream_t s);

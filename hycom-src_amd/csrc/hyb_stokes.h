@@ -29,11 +29,10 @@ struct PiStokes {
   static constexpr bool kRawThk = false;
   const double* sdzi;
   double pbot;
-  HYB_HD double first() const { return 0.0; }
-  HYB_HD double raw(int x) const { return sdzi[x - 1]; }
+  HYB_HD double first(int64_t) const { return 0.0; }
+  HYB_HD double raw(int x, int64_t) const { return sdzi[x - 1]; }
   HYB_HD double comb(double, double r) const { return dmin(r, pbot); }
-  HYB_HD double nextfrom(int x, double pix) const { return comb(pix, raw(x)); }
-  HYB_HD double thk(int) const { return 0.0; }
+  HYB_HD double thk(int, int64_t) const { return 0.0; }
 };
 
 // New interfaces prsf(1) = 0, prsf(k+1) = min(prsf(k) + dp(k), p(kk+1))
@@ -72,15 +71,20 @@ struct StokesBlend {
   double x, y, w0, w1;
   HYB_HD operator double() const { return w0 * x + w1 * y; }
 };
+HYB_HD void slot_arrived(StokesBlend& s) {
+  s.x = arrived(s.x);
+  s.y = arrived(s.y);
+}
 struct StokesRow {  // one field of one column; level stride 2S, snapshot 2 at +S
   const double* a;
   int64_t S;
   double w0, w1;
-  HYB_HD StokesBlend operator[](int64_t i) const {
-    const int64_t o = 2 * i;  // i = (k-1)*S as walk_core forms it
-    return StokesBlend{a[o], a[o + S], w0, w1};
-  }
 };
+// off = (k-1)*S as walk_core forms it
+HYB_HD StokesBlend row_at(const StokesRow& r, int64_t off, int64_t c) {
+  const double* a = r.a + 2 * off;
+  return StokesBlend{a[c], (a + r.S)[c], r.w0, r.w1};
+}
 struct StokesFields {
   StokesRow row[2];
   HYB_HD const StokesRow& operator[](int f) const { return row[f]; }
@@ -94,12 +98,13 @@ HYB_HDI void stokes_column(const KStokes& Q, int64_t c0) {
   const double pbot = Q.p[c0 + S * (int64_t)Q.kk];
   PiStokes pi{Q.sdzi, pbot};
   PoStokes po(Q.dp + c0 + S * (int64_t)Q.kk * (Q.n - 1), S, pbot, Q.kk);
-  const StokesFields fp{{StokesRow{Q.usdz + c0, S, Q.ws0, Q.ws1},
-                         StokesRow{Q.vsdz + c0, S, Q.ws0, Q.ws1}}};
-  double* op[2] = {Q.usdp + c0, Q.vsdp + c0};
+  const StokesFields fp{{StokesRow{Q.usdz, S, Q.ws0, Q.ws1},
+                         StokesRow{Q.vsdz, S, Q.ws0, Q.ws1}}};
+  double* op[2] = {Q.usdp, Q.vsdp};
   FieldSink<2> sink{op, 2, nullptr, 0.0, S};
   const double zx = dmin(Q.sdzi[Q.nsdzi - 1], pbot);
-  walk_core<1, 2, PD, false, true>(Q.nsdzi, zx, pi, po, sink, fp, 2, Q.nsdzi, 0ull, S, Q.kk);
+  walk_core<1, 2, PD, false, true, false, false>(Q.nsdzi, zx, pi, po, sink, fp, 2, Q.nsdzi, 0ull, S, Q.kk,
+                                    c0);
 }
 
 }  // namespace hyb

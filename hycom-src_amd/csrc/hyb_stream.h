@@ -766,44 +766,70 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
 // Sources of the old interfaces pi(x) for walk_core: pi(1), then pi(x+1)
 // from pi(x) (the walk asks for them in increasing x, and scans ahead).
 // ---------------------------------------------------------------------
-// raw(x) is the memory word that gives pi(x+1) from pi(x) through comb(),
-// so a walk can issue it early.
+// raw(x, c) is the memory word of column c that gives pi(x+1) from pi(x)
+// through comb(), so a walk can issue it early.  Pointers are those of the
+// level's first column, uniform over the wave, and c the column's offset, one
+// per lane: a pointer kept per lane costs two registers for every array.
 // kRawThk: the walk takes the old thicknesses dprs(x) from thk(x) as
 // stored instead of as differences of the interfaces.
 struct PiArray {  // p-columns: the overturned interfaces left by regrid_stream
   static constexpr bool kRawThk = false;
   const double* pres;
   int64_t S;
-  HYB_HD double thk(int) const { return 0.0; }
-  HYB_HD double first() const { return pres[0]; }
-  HYB_HD double raw(int x) const { return pres[(int64_t)x * S]; }
+  HYB_HD double thk(int, int64_t) const { return 0.0; }
+  HYB_HD double first(int64_t c) const { return pres[c]; }
+  HYB_HD double raw(int x, int64_t c) const { return (pres + (int64_t)x * S)[c]; }
   HYB_HD double comb(double, double r) const { return r; }
-  HYB_HD double nextfrom(int x, double pix) const { return comb(pix, raw(x)); }
 };
 struct PiSum {  // u/v points: running sums of the old dpu (hybgen.F90:171-195)
   static constexpr bool kRawThk = false;
   const double* dpu;
   int64_t S;
-  HYB_HD double thk(int) const { return 0.0; }
-  HYB_HD double first() const { return 0.0; }
-  HYB_HD double raw(int x) const { return dpu[(int64_t)(x - 1) * S]; }
+  HYB_HD double thk(int, int64_t) const { return 0.0; }
+  HYB_HD double first(int64_t) const { return 0.0; }
+  HYB_HD double raw(int x, int64_t c) const { return (dpu + (int64_t)(x - 1) * S)[c]; }
   HYB_HD double comb(double pix, double r) const { return pix + r; }
-  HYB_HD double nextfrom(int x, double pix) const { return comb(pix, raw(x)); }
 };
 // hybgencj (hybgen.F90:1909-2274): the old interfaces are running sums of
 // the old dp(m), kept in the workspace, and the old thicknesses are dp(m)
 // itself (hybgencj passes dprs(k) = dp(k,m), not pres(k+1)-pres(k)).
 struct PiRa {
   static constexpr bool kRawThk = true;
-  const double* pres;  // the running sums, level 1 of the column
-  const double* dpm;   // dp(:,m), level 1 of the column
+  const double* pres;  // the running sums, level 1
+  const double* dpm;   // dp(:,m), level 1
   int64_t S;
-  HYB_HD double first() const { return pres[0]; }
-  HYB_HD double raw(int x) const { return pres[(int64_t)x * S]; }
+  HYB_HD double first(int64_t c) const { return pres[c]; }
+  HYB_HD double raw(int x, int64_t c) const { return (pres + (int64_t)x * S)[c]; }
   HYB_HD double comb(double, double r) const { return r; }
-  HYB_HD double nextfrom(int x, double pix) const { return comb(pix, raw(x)); }
-  HYB_HD double thk(int x) const { return dpm[(int64_t)(x - 1) * S]; }
+  HYB_HD double thk(int x, int64_t c) const { return (dpm + (int64_t)(x - 1) * S)[c]; }
 };
+
+// x in a register of its own: a look-ahead value leaves its slot by this
+// move, so the slot is free for the next load (without it the allocator
+// keeps x in the slot, loads the next value elsewhere, and copies it back
+// at the end of the turn, waiting for the load there).
+HYB_HD double leave_slot(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y;
+  asm volatile("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
+  return y;
+#else
+  return x;
+#endif
+}
+
+// x, a value just loaded, waited for here: used where a load is rare and
+// sits in a branch, so that the wait stays in the branch too.  (Left to its
+// use after the branches join, the wait is for every outstanding load and is
+// paid whether the branch was taken or not.)
+HYB_HD double arrived(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(x));
+#endif
+  return x;
+}
+// the same for a look-ahead slot in place (StokesBlend has its own)
+HYB_HD void slot_arrived(double& x) { x = arrived(x); }
 
 // New interfaces prsf(k): p-columns keep them in the lane's LDS column
 // (LaneRow); u/v points keep the new thicknesses there and sum them as
@@ -830,12 +856,12 @@ struct PoSum {
 
 // The same prsf(k) without the LDS column: the new thicknesses are formed
 // again from p at the two neighbouring p-points as the walk asks for them
-// (the operations of the first pass of uv_stream, so the same bits).  The
-// p levels are loaded A levels ahead of the request, unconditionally (the
-// index clamped into the column), so the loads are issued without a
-// branch and have the work of A requests to arrive.
-template <int A>
-struct PoRecomputeT {
+// (the operations of the first pass of uv_stream, so the same bits).  Two
+// levels are held ahead of the request: one arrived (ra, rb) and one on its
+// way (qa, qb).  The walk calls ready() and then load() once per layer, with
+// its own look-ahead loads: everything loaded in a layer is waited for in
+// one place, a layer later, and a request finds its words in registers.
+struct PoRecompute {
   const double* p0;
   const double* p1;
   int64_t S;
@@ -843,56 +869,87 @@ struct PoRecomputeT {
   int k1;                                // kk+1, the deepest level
   double prv = 0.0, cur = 0.0, b = 0.0;  // prsf(k-1), prsf(k), min(depthu, p-mean at k)
   double dl = 0.0;                       // the new thickness of layer k-1 (cur = prv + dl)
-  double q0[A], q1[A];                   // p at levels k+1..k+A of both points, loaded ahead
-  int64_t at = 0;                        // offset of level k+A, clamped into the column
+  double ra = 0.0, rb = 0.0, qa = 0.0, qb = 0.0;
+  bool has_r = false, has_q = false;
+  int64_t c0;                            // the column's offset in a level
+  int64_t at = 0;                        // offset of the last level loaded, c0 included
+  int x = 0;                             // that level, from 0; clamped to kk
   int k = 0;                             // 0 until the first request
-  HYB_HD PoRecomputeT(const double* a0, const double* a1, int64_t s, double du, int kk)
-      : p0(a0), p1(a1), S(s), depthu(du), k1(kk + 1) {
-#pragma unroll
-    for (int q = 0; q < A; q++) q0[q] = q1[q] = 0.0;
+  HYB_HD PoRecompute(const double* a0, const double* a1, int64_t s, double du, int kk, int64_t c)
+      : p0(a0), p1(a1), S(s), depthu(du), k1(kk + 1), c0(c) {}
+  HYB_HD void next() {
+    if (x < k1 - 1) {
+      x++;
+      at += S;
+    }
+  }
+  HYB_HD void step(double a0, double a1) {
+    const double a = dmin(depthu, 0.5 * (a0 + a1));
+    const double d = dmax(0.0, a - b);
+    b = a;
+    prv = cur;
+    cur = cur + d;
+    dl = d;
+    k++;
   }
   HYB_HD double operator()(int kq) {
     if (kq == 1 || k == 0) {
       prv = 0.0;
       cur = 0.0;
       dl = 0.0;
-      b = dmin(depthu, 0.5 * (p0[0] + p1[0]));
+      b = dmin(depthu, 0.5 * (p0[c0] + p1[c0]));
       k = 1;
-#pragma unroll
-      for (int q = 0; q < A; q++) {
-        at = (int64_t)(1 + q < k1 ? 1 + q : k1 - 1) * S;
-        q0[q] = p0[at];
-        q1[q] = p1[at];
-      }
+      x = 0;
+      at = c0;
+      next();
+      ra = p0[at];
+      rb = p1[at];
+      next();
+      qa = p0[at];
+      qb = p1[at];
+      has_r = has_q = true;
     }
     while (k < kq) {
-      const double a = dmin(depthu, 0.5 * (q0[0] + q1[0]));
-      const double d = dmax(0.0, a - b);
-      b = a;
-      prv = cur;
-      cur = cur + d;
-      dl = d;
-      k++;
-#pragma unroll
-      for (int q = 0; q < A - 1; q++) {
-        q0[q] = q0[q + 1];
-        q1[q] = q1[q + 1];
+      double a0 = ra, a1 = rb;
+      if (!has_r) {
+        if (!has_q) {
+          next();
+          qa = p0[at];
+          qb = p1[at];
+        }
+        a0 = arrived(qa);
+        a1 = arrived(qb);
+        has_q = false;
       }
-      if (k + A - 1 < k1) at += S;
-      q0[A - 1] = p0[at];
-      q1[A - 1] = p1[at];
+      has_r = false;
+      step(a0, a1);
     }
     return cur;
   }
+  HYB_HD void ready() {
+    if (!has_r && has_q) {
+      ra = leave_slot(qa);
+      rb = leave_slot(qb);
+      has_r = true;
+      has_q = false;
+    }
+  }
+  HYB_HD void load() {
+    if (!has_q) {
+      next();
+      qa = p0[at];
+      qb = p1[at];
+      has_q = true;
+    }
+  }
 };
-using PoRecompute = PoRecomputeT<1>;
 template <class PO>
 struct is_recompute : std::false_type {};
-template <int A>
-struct is_recompute<PoRecomputeT<A>> : std::true_type {};
+template <>
+struct is_recompute<PoRecompute> : std::true_type {};
 
 // Output sinks.  emit(kc, at, v, certain, thick): v[f] is output kc of field
-// f before the clamp, at its offset (kc-1)*S from level 1; certain means it lies inside the range of the input
+// f before the clamp, at its offset (kc-1)*S + c0 from level 1; certain means it lies inside the range of the input
 // levels read so far, so the clamp against the whole column cannot change
 // it.  fixup() clamps the others once the column range is known.
 // NT: outputs written with non-temporal stores (streamed past the caches)
@@ -925,7 +982,7 @@ struct FieldSink {  // T, S, tracers; th3d from T and S (hybgen.F90:1549-1569)
   }
   // outputs kc..KN all take v (clamped); k is uniform over the wave, so a
   // level is written as one row
-  HYB_HD void tail(int kc, int KN, const double* v, uint64_t) {
+  HYB_HD void tail(int kc, int KN, const double* v, uint64_t, int64_t c0) {
     double th = 0.0;
     if constexpr (NF >= 2)
       if (th3d) th = sig(v[0], v[1]) - thbase;
@@ -933,15 +990,15 @@ struct FieldSink {  // T, S, tracers; th3d from T and S (hybgen.F90:1549-1569)
       if (k < kc) continue;
 #pragma unroll
       for (int f = 0; f < NF; f++)
-        if (f < nf) put(fp[f] + (int64_t)(k - 1) * S, v[f]);
+        if (f < nf) put(fp[f] + (int64_t)(k - 1) * S + c0, v[f]);
       if constexpr (NF >= 2)
-        if (th3d) put(th3d + (int64_t)(k - 1) * S, th);
+        if (th3d) put(th3d + (int64_t)(k - 1) * S + c0, th);
     }
   }
   // clamp to [smin, smax] the outputs outside [lo, hi] (lo = smin and
   // hi = smax except in the mixed form, see walk_core)
   HYB_HD void fixup(const double* lo, const double* hi, const double* smin,
-                    const double* smax) {
+                    const double* smax, int64_t c0) {
     while (fix) {
       const int k = __builtin_ctzll(fix) + 1;
       fix &= fix - 1;
@@ -950,15 +1007,15 @@ struct FieldSink {  // T, S, tracers; th3d from T and S (hybgen.F90:1549-1569)
       for (int f = 0; f < NF; f++) {
         v[f] = 0.0;
         if (f < nf) {
-          double x = fp[f][(int64_t)(k - 1) * S];
+          double x = fp[f][(int64_t)(k - 1) * S + c0];
           x = (x < lo[f]) ? smin[f] : x;
           x = (x > hi[f]) ? smax[f] : x;
-          fp[f][(int64_t)(k - 1) * S] = x;
+          fp[f][(int64_t)(k - 1) * S + c0] = x;
           v[f] = x;
         }
       }
       if constexpr (NF >= 2)
-        if (th3d) th3d[(int64_t)(k - 1) * S] = sig(v[0], v[1]) - thbase;
+        if (th3d) th3d[(int64_t)(k - 1) * S + c0] = sig(v[0], v[1]) - thbase;
     }
   }
 };
@@ -986,23 +1043,46 @@ struct UvSink {  // u or v with the thin-layer rule (hybgen.F90:1858-1865)
     }
     if constexpr (is_recompute<PO>::value) dpn[at] = po->dl;
   }
-  // outputs kc..KN all take v (clamped), by the rule of emit
-  HYB_HD void tail(int kc, int KN, const double* v, uint64_t thick) {
-    for (int k = 1; k <= KN; k++) {
-      if (k < kc) continue;
-      (void)(*po)(k + 1);
-      emit(k, (int64_t)(k - 1) * S, v, true, (thick >> (k - 1)) & 1ull);
+  // outputs kc..KN all take v (clamped), by the rule of emit.  The levels
+  // of p are loaded eight at a time (po stands at level kc).
+  HYB_HD void tail(int kc, int KN, const double* v, uint64_t thick, int64_t c0) {
+    if constexpr (is_recompute<PO>::value) {
+      constexpr int B = 8;
+#pragma unroll 1
+      for (int k0 = 1; k0 <= KN; k0 += B) {
+        if (k0 + B - 1 < kc) continue;
+        double a0[B], a1[B];
+#pragma unroll
+        for (int q = 0; q < B; q++) {
+          const int64_t o = (int64_t)(k0 + q < KN ? k0 + q : KN) * S;
+          a0[q] = (po->p0 + o)[c0];
+          a1[q] = (po->p1 + o)[c0];
+        }
+#pragma unroll
+        for (int q = 0; q < B; q++) {
+          const int k = k0 + q;
+          if (k < kc || k > KN) continue;
+          po->step(a0[q], a1[q]);
+          emit(k, (int64_t)(k - 1) * S + c0, v, true, (thick >> (k - 1)) & 1ull);
+        }
+      }
+    } else {
+      for (int k = 1; k <= KN; k++) {
+        if (k < kc) continue;
+        (void)(*po)(k + 1);
+        emit(k, (int64_t)(k - 1) * S + c0, v, true, (thick >> (k - 1)) & 1ull);
+      }
     }
   }
   HYB_HD void fixup(const double* lo, const double* hi, const double* smin,
-                    const double* smax) {
+                    const double* smax, int64_t c0) {
     while (fix) {
       const int k = __builtin_ctzll(fix) + 1;
       fix &= fix - 1;
-      double x = uu[(int64_t)(k - 1) * S];
+      double x = uu[(int64_t)(k - 1) * S + c0];
       x = (x < lo[0]) ? smin[0] : x;
       x = (x > hi[0]) ? smax[0] : x;
-      uu[(int64_t)(k - 1) * S] = x;
+      uu[(int64_t)(k - 1) * S + c0] = x;
     }
   }
 };
@@ -1020,20 +1100,6 @@ struct CoefState {
   R zw3l[NF];                             // WENO interface value zw3(l)
   R qdpjp_l, wq_l;                        // PPM qdpjp(l); WENO 1/(dp(l)+dp(l+1))
 };
-
-// x in a register of its own: a look-ahead value leaves its slot by this
-// move, so the slot is free for the next load (without it the allocator
-// keeps x in the slot, loads the next value elsewhere, and copies it back
-// at the end of the turn, waiting for the load there).
-HYB_HD double leave_slot(double x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  double y;
-  asm("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
-  return y;
-#else
-  return x;
-#endif
-}
 
 // sign(min(|a|,|b|,|c|), b) for finite or infinite a, b, c, in three
 // instructions on the device (NaN operands do not reach a use of it: the
@@ -1266,22 +1332,31 @@ __attribute__((always_inline)) HYB_HD void coef_layer(
 // ---------------------------------------------------------------------
 // remap of up to NF fields of one column in one walk over the old layers
 // (hybgen_{pcm,plm,ppm,weno}_{coefs,remap}).  fp[f] points at level 1 of
-// field f (stride S); levels > kp take level kp's value (the massless
+// field f (stride S), c0 is the column's offset in a level; levels > kp take level kp's value (the massless
 // fill); zx = pi(K+1).  PD levels of every field (and of the old
 // interfaces) are loaded ahead of the window, to cover memory latency.
-// K old layers, KO new ones (KO = 0: K).  CDPI: the PLM slopes are taken
+// K old layers, KO new ones (KO = 0: K).  FILL off: kp = K, no fill.  CDPI: the PLM slopes are taken
 // on dpi = max(dprs, thin) instead of dprs (mod_stokes.F90:683-684 passes
-// dpi to hybgen_plm_coefs; hybgen.F90:1535 passes dprs).  fp[f][i] is a
+// dpi to hybgen_plm_coefs; hybgen.F90:1535 passes dprs).  row_at(fp[f]) is a
 // double, or a value that converts to one when the level enters the window
 // (a blend of two stored words, so the loads stay outstanding until then).
 // ---------------------------------------------------------------------
+HYB_HD double row_at(const double* p, int64_t off, int64_t c) { return (p + off)[c]; }
+// c, which the compiler takes as changed: base + c is then formed where it is
+// used, from a uniform base, and not kept in two registers per array
+HYB_HD int64_t opaque(int64_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(c));
+#endif
+  return c;
+}
 template <int METHOD, int NF, int PD, bool FAST = false, bool CDPI = false, bool FDIV = false,
-          class PI, class PO, class SINK, class FP>
+          bool FILL = true, class PI, class PO, class SINK, class FP>
 HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const FP& fp,
-                      int nf, int kp, uint64_t lcm, int64_t S, int KO = 0) {
+                      int nf, int kp, uint64_t lcm, int64_t S, int KO = 0, int64_t c0 = 0) {
   constexpr int PQ = PD > 0 ? PD : 1;
   const int KN = KO > 0 ? KO : K;
-  using RawT = typename std::decay<decltype(fp[0][0])>::type;
+  using RawT = decltype(row_at(fp[0], (int64_t)0, (int64_t)0));
   using CR = typename std::conditional<FAST, float, double>::type;
   const double thin = kDpthin;
   const double dsmll = 1.0e-8;
@@ -1295,7 +1370,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
 
   // per-field state
   double s0[NF], s1[NF], s2[NF], s3[NF];  // s(l-1), s(l), s(l+1), s(l+2)
-  double smin[NF], smax[NF], skp[NF], sfirst[NF];
+  double smin[NF], smax[NF], skp[NF];
   double acc[NF], ov[NF], prev[NF];
   // FAST (the mixed form): each output's sum of piece integrals is
   // compensated (TwoSum: acc + accc), as the sums that set conservation
@@ -1313,8 +1388,8 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
   // fold(f, x, r): level x enters the column in order, r being its stored
   // value (ignored below kp); idempotent, so a level may be folded again
   auto fold = [&](int f, int x, double r) -> double {
-    const double v = (x <= kp) ? r : skp[f];
-    if (x == kp) skp[f] = v;
+    const double v = (!FILL || x <= kp) ? r : skp[f];
+    if (FILL && x == kp) skp[f] = v;
     if (x == 1) {
       smin[f] = v;
       smax[f] = v;
@@ -1325,7 +1400,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     return v;
   };
   auto load = [&](int f, int x) -> double {
-    return fold(f, x, (x <= kp) ? static_cast<double>(fp[f][(int64_t)(x - 1) * S]) : 0.0);
+    return fold(f, x, (x <= kp) ? static_cast<double>(row_at(fp[f], (int64_t)(x - 1) * S, c0)) : 0.0);
   };
   // The first window: every load is issued before any is used (levels
   // clamped into the column; a value below kp or the bottom is not used).
@@ -1334,33 +1409,33 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
 #pragma unroll
   for (int f = 0; f < NF; f++) {
     if (f < nf) {
-      r1[f] = fp[f][0];
-      r2[f] = fp[f][(int64_t)(lx(2) - 1) * S];
-      r3[f] = fp[f][(int64_t)(lx(3) - 1) * S];
+      r1[f] = row_at(fp[f], 0, c0);
+      r2[f] = row_at(fp[f], (int64_t)(lx(2) - 1) * S, c0);
+      r3[f] = row_at(fp[f], (int64_t)(lx(3) - 1) * S, c0);
 #pragma unroll
-      for (int q = 0; q < PD; q++) sq[f][q] = fp[f][(int64_t)(lx(4 + q) - 1) * S];
+      for (int q = 0; q < PD; q++) sq[f][q] = row_at(fp[f], (int64_t)(lx(4 + q) - 1) * S, c0);
     }
   }
-  const double pr1 = pi.raw(1), pr2 = pi.raw(lx(2)), pr3 = pi.raw(lx(3));
+  const double pr1 = pi.raw(1, c0), pr2 = pi.raw(lx(2), c0), pr3 = pi.raw(lx(3), c0);
 #pragma unroll
-  for (int q = 0; q < PD; q++) prq[q] = pi.raw(lx(4 + q));
+  for (int q = 0; q < PD; q++) prq[q] = pi.raw(lx(4 + q), c0);
   if constexpr (RAWT) {
-    tv1 = pi.thk(1);
-    tv2 = pi.thk(lx(2));
-    tv3 = pi.thk(lx(3));
+    tv1 = pi.thk(1, c0);
+    tv2 = pi.thk(lx(2), c0);
+    tv3 = pi.thk(lx(3), c0);
 #pragma unroll
-    for (int q = 0; q < PQ; q++) tq[q] = pi.thk(lx(4 + q));
+    for (int q = 0; q < PQ; q++) tq[q] = pi.thk(lx(4 + q), c0);
   }
   xl = 4 + PD;
   // interfaces pi(l-1..l+3) at l = 1
-  double pv0 = 0.0, pv1 = pi.first(), pv2 = 0.0, pv3 = 0.0, pv4 = 0.0;
+  double pv0 = 0.0, pv1 = pi.first(c0), pv2 = 0.0, pv3 = 0.0, pv4 = 0.0;
   pv2 = pi.comb(pv1, pr1);
   if (K >= 2) pv3 = pi.comb(pv2, pr2);
   if (K >= 3) pv4 = pi.comb(pv3, pr3);
 #pragma unroll
   for (int f = 0; f < NF; f++) {
     s0[f] = s1[f] = s2[f] = s3[f] = 0.0;
-    smin[f] = smax[f] = skp[f] = sfirst[f] = 0.0;
+    smin[f] = smax[f] = skp[f] = 0.0;
     acc[f] = ov[f] = prev[f] = accc[f] = 0.0;
     cst.asc[f] = cst.alc[f] = 0.0;
     cst.wc1[f] = cst.wc2[f] = cst.wz1[f] = cst.wz2[f] = cst.zw3l[f] = 0.0;
@@ -1368,7 +1443,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
       s1[f] = fold(f, 1, static_cast<double>(r1[f]));
       if (K >= 2) s2[f] = fold(f, 2, static_cast<double>(r2[f]));
       if (K >= 3) s3[f] = fold(f, 3, static_cast<double>(r3[f]));
-      sfirst[f] = s1[f];
+      prev[f] = s1[f];  // a thin first output takes s(1)
       if (METHOD == 2) cst.alc[f] = (CR)s1[f];  // al(1) = s(1)
       if (METHOD == 3) {                        // first sweep of layer 1
         cst.wc1[f] = (CR)s1[f];
@@ -1404,15 +1479,15 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     while (lt_c < K && pn < zb0) {
       lt_c++;
       pc = pn;
-      if (lt_c < K) pn = pi.nextfrom(lt_c, pc);
+      if (lt_c < K) pn = pi.comb(pc, pi.raw(lt_c, c0));
     }
   }
   double zt_c = zb0;
   int kc = 1;
-  int64_t kat = 0;  // (kc-1)*S
+  int64_t kat = c0;  // offset of output kc: (kc-1)*S + c0
   bool accon = false, acc_thin = false;
   int lb_act = 0;
-  double zt_act = 0.0, zb_act = 0.0;
+  double zb_act = 0.0;  // bottom of the output in progress (its top is zt_c)
 
   // The clamp to the column range (e.g. 2836-2837).  The mixed form lets
   // values within a slack of 2^-20 of the range's magnitude stand (in the
@@ -1543,10 +1618,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
         double v[NF];
         if (acc_thin) {
 #pragma unroll
-          for (int f = 0; f < NF; f++) {
-            const double a = prev[f], b = sfirst[f];
-            v[f] = (kc != 1) ? a : b;
-          }
+          for (int f = 0; f < NF; f++) v[f] = prev[f];
         } else {
           const double xb = xof(zb_act);
           const double dpb = zb_act - pil;
@@ -1563,7 +1635,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
             qb2 = qb1 - 1.0 + xb;
             qb0 = 1.0 - qb1 - qb2;
           }
-          const double dz = zb_act - zt_act;
+          const double dz = zb_act - zt_c;
           const double rdz = FAST ? frcp64(dz) : 0.0;
           const Rcp64 rz = FD64 ? rcp64(dz) : Rcp64{0.0, 0.0};
 #pragma unroll
@@ -1616,10 +1688,7 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
           double v[NF];
           if (thn) {
 #pragma unroll
-            for (int f = 0; f < NF; f++) {
-              const double a = prev[f], b = sfirst[f];
-              v[f] = (kc != 1) ? a : b;
-            }
+            for (int f = 0; f < NF; f++) v[f] = prev[f];
           } else if (METHOD == 0) {
 #pragma unroll
             for (int f = 0; f < NF; f++) v[f] = s1[f];
@@ -1676,14 +1745,13 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
             lb = l + 3;
             double pc = pv4;  // pi(l+3)
             while (lb < K) {
-              const double pn = pi.nextfrom(lb, pc);
+              const double pn = pi.comb(pc, pi.raw(lb, c0));
               if (!(pn < zb)) break;
               lb++;
               pc = pn;
             }
           }
           lb_act = lb;
-          zt_act = zt;
           zb_act = zb;
           acc_thin = thn;
           accon = true;
@@ -1711,9 +1779,10 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
                 double o = s1[f];
                 if (mid != l) {
                   const double w2 = s2[f], w3 = s3[f], wk = skp[f];
-                  o = mid == l + 1 ? w2 : (mid == l + 2 ? w3 : wk);
-                  if (mid > l + 2 && kp > l + 2)
-                    o = static_cast<double>(fp[f][(int64_t)((mid < kp ? mid : kp) - 1) * S]);
+                  o = mid == l + 1 ? w2 : ((!FILL || mid == l + 2) ? w3 : wk);
+                  if (mid > l + 2 && (!FILL || kp > l + 2))
+                    o = arrived(static_cast<double>(
+                        row_at(fp[f], (int64_t)((mid < kp ? mid : kp) - 1) * S, c0)));
                 }
                 ov[f] = o;
                 accc[f] = 0.0;
@@ -1751,15 +1820,28 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
 #if defined(__HIP_DEVICE_COMPILE__)
     __builtin_amdgcn_s_setprio(2);
 #endif
+    // Everything loaded ahead is waited for here, before any of the next
+    // loads is issued, and whether or not it is used: a slot that might still
+    // be in flight on some path would make the compiler wait for the newest
+    // loads when it reuses the slot's registers.
+    double pnew = 0.0;
+    if constexpr (is_recompute<PO>::value) po.ready();
+    if constexpr (PD > 0) {
+      pnew = leave_slot(prq[B]);
+#pragma unroll
+      for (int f = 0; f < NF; f++) slot_arrived(sq[f][B]);
+    }
+    if constexpr (RAWT) tq[B] = arrived(tq[B]);
+    c0 = opaque(c0);
     const double top = pv4;
     pv0 = pv1;
     pv1 = pv2;
     pv2 = pv3;
     pv3 = top;
     if (PD == 0) {
-      pv4 = (l + 4 <= K + 1) ? pi.nextfrom(l + 3, top) : 0.0;
+      pv4 = (l + 4 <= K + 1) ? pi.comb(top, pi.raw(l + 3, c0)) : 0.0;
     } else {
-      pv4 = (l + 4 <= K + 1) ? pi.comb(top, leave_slot(prq[B])) : 0.0;
+      pv4 = (l + 4 <= K + 1) ? pi.comb(top, pnew) : 0.0;
     }
     if (l + 3 <= K && dmax(pv4 - pv3, thin) > thin) thick |= 1ull << (l + 2);
     if constexpr (RAWT) {
@@ -1782,15 +1864,16 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     // slot B is free: level l+3+PQ goes into it.  Clamped into the column
     // and unconditional for the interfaces; the fields' levels below kp are
     // not loaded (the fill takes their place).
+    if constexpr (is_recompute<PO>::value) po.load();
     if (PD > 0 || RAWT) {
       const int xn = l + 3 + PQ;
       const int xk = xn < K ? xn : K;
-      if (PD > 0) prq[B] = pi.raw(xk);
-      if constexpr (RAWT) tq[B] = pi.thk(xk);
+      if (PD > 0) prq[B] = pi.raw(xk, c0);
+      if constexpr (RAWT) tq[B] = pi.thk(xk, c0);
       if (PD > 0 && xn <= kp) {
 #pragma unroll
         for (int f = 0; f < NF; f++)
-          if (f < nf) sq[f][B] = fp[f][(int64_t)(xn - 1) * S];
+          if (f < nf) sq[f][B] = row_at(fp[f], (int64_t)(xn - 1) * S, c0);
       }
     }
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1823,15 +1906,14 @@ HYB_HDI void walk_core(int K, double zx, const PI& pi, PO& po, SINK& sink, const
     double tl[NF];
 #pragma unroll
     for (int f = 0; f < NF; f++) {
-      const double a = prev[f], b = sfirst[f];
-      double x = (kc != 1) ? a : b;
+      double x = prev[f];
       x = (x < lo[f]) ? smin[f] : x;
       x = (x > hi[f]) ? smax[f] : x;
       tl[f] = x;
     }
-    sink.tail(kc, KN, tl, thick);
+    sink.tail(kc, KN, tl, thick, c0);
   }
-  sink.fixup(lo, hi, smin, smax);
+  sink.fixup(lo, hi, smin, smax, c0);
 }
 
 // ---------------------------------------------------------------------
@@ -1850,13 +1932,15 @@ HYB_HDI void remap_walk_pi(const KParams& P, const View& V, int64_t c0, int n, i
 #pragma unroll
   for (int f = 0; f < NW; f++) {
     const int g = g0 + f;
-    if (g == 0) fp[f] = V.temp + c0 + lev4(V, 1, n);
-    else if (g == 1) fp[f] = V.saln + c0 + lev4(V, 1, n);
-    else fp[f] = V.tracer + c0 + levt(V, 1, n, g - 1);
+    if (g == 0) fp[f] = V.temp + lev4(V, 1, n);
+    else if (g == 1) fp[f] = V.saln + lev4(V, 1, n);
+    else fp[f] = V.tracer + levt(V, 1, n, g - 1);
   }
-  double* th = (g0 == 0) ? V.th3d + c0 + lev4(V, 1, n) : nullptr;
+  double* th = (g0 == 0) ? V.th3d + lev4(V, 1, n) : nullptr;
   FieldSink<NW, NT> sink{dst ? dst : fp, NW, th, P.thbase, S};
-  walk_core<METHOD, NW, PD, FAST, false, true>(K, zx, pi, po, sink, fp, NW, kp, lcm, S, KO);
+  // a source with stored thicknesses is the RA branch, which has no fill
+  walk_core<METHOD, NW, PD, FAST, false, true, !PI::kRawThk>(K, zx, pi, po, sink, fp, NW, kp, lcm, S,
+                                                             KO, c0);
 }
 template <int METHOD, int NW, int PD, bool FAST, bool NT, class PO>
 HYB_HDI void remap_walk(const KParams& P, const View& V, int64_t c0, int n, int g0, int K,
@@ -1885,8 +1969,8 @@ HYB_HDI void remap_fields(const KParams& P, const View& V, const Scratch& W, int
   if (kpw & kUnsafe) return;
   const int kp = kpw & 0xffff;
   const uint64_t lcm = W.lcm[c0];
-  const double* pres = W.pres + c0;
-  const double zx = pres[(int64_t)K * S];
+  const double* pres = W.pres;
+  const double zx = pres[(int64_t)K * S + c0];
   const int nfields = 2 + P.ntracr;
   int g0 = 0;
   for (; g0 + NF <= nfields; g0 += NF)
@@ -2020,8 +2104,8 @@ HYB_HDI void remap_pair(const KParams& P, const View& V, const Scratch& W, int64
   const int K = P.kk;
   const int kp = kpw & 0xffff;
   const uint64_t lcm = W.lcm[c0];
-  const double* pres = W.pres + c0;
-  const double zx = pres[(int64_t)K * V.NIJ];
+  const double* pres = W.pres;
+  const double zx = pres[(int64_t)K * V.NIJ + c0];
   const int g0 = 2 * q, r = 2 + P.ntracr - g0;
   if (r >= 2)
     remap_walk<METHOD, 2, PD, FAST, false>(P, V, c0, n, g0, K, zx, pres, kp, lcm, po);
@@ -2042,7 +2126,7 @@ HYB_HDI void ra_walk(const KParams& P, const View& V, const Scratch& W, int64_t 
   const int64_t S = V.NIJ;
   double* dst[NW];
 #pragma unroll
-  for (int f = 0; f < NW; f++) dst[f] = W.ras + c0 + (int64_t)f * K * S;
+  for (int f = 0; f < NW; f++) dst[f] = W.ras + (int64_t)f * K * S;
   remap_walk_pi<METHOD, NW, PD, false, false>(P, V, c0, m, g0, K, zx, pi, K, lcm, po, K, dst);
 #pragma unroll
   for (int f = 0; f < NW; f++) {
@@ -2050,7 +2134,7 @@ HYB_HDI void ra_walk(const KParams& P, const View& V, const Scratch& W, int64_t 
     double* fp = (g == 0) ? V.temp + c0 + lev4(V, 1, m)
                : (g == 1) ? V.saln + c0 + lev4(V, 1, m)
                           : V.tracer + c0 + levt(V, 1, m, g - 1);
-    stage_column(fp, 0, dst[f], S, K, S);
+    stage_column(fp, 0, dst[f] + c0, S, K, S);
   }
 }
 
@@ -2205,7 +2289,7 @@ HYB_HDI bool ra_stream(const KParams& P, const View& V, const Scratch& W, int i,
   const bool staged = have && cand <= zlast;
   if (!tame || (staged && !W.ras)) return false;
   StagedInterfaces po{row, ld, K + 1, 0.0, ps};
-  PiRa pi{pres, dpm, S};
+  PiRa pi{W.pres, V.dp + lev4(V, 1, m), S};
   const int nfields = 2 + P.ntracr;
   int g0 = 0;
   for (; g0 + NF <= nfields; g0 += NF)
@@ -2267,7 +2351,6 @@ HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bo
   const int64_t S = V.NIJ;
   const int64_t cn = isv ? ij_of(V, i, j - 1) : ij_of(V, i - 1, j);
   double* dpu = (isv ? V.dpv : V.dpu) + c0 + lev4(V, 1, nl);
-  double* uu = (isv ? V.v : V.u) + c0 + lev4(V, 1, nl);
   double* pu = (isv ? V.pv : V.pu) + c0;
   const double depthu = (isv ? V.depthv : V.depthu)[c0];
   const double ub = (isv ? V.vbavg : V.ubavg)[c0 + lev(V, nl)];
@@ -2337,16 +2420,21 @@ HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bo
   }
   const double zx = q2;
   if ((have && cand < zx) || !tame) return false;
-  PiSum pi{dpu, S};
-  double* fp[1] = {uu};
+  double* dpu1 = (isv ? V.dpv : V.dpu) + lev4(V, 1, nl);  // level 1
+  double* uu1 = (isv ? V.v : V.u) + lev4(V, 1, nl);
+  PiSum pi{dpu1, S};
+  double* fp[1] = {uu1};
   if (RECOMP) {
-    PoRecompute po(p0, p1, S, depthu, K);
-    UvSink<PoRecompute> sink{uu, S, ub, pr, &po, 0ull, dpu};
-    walk_core<METHOD, 1, PD, MIXED, false, true>(K, zx, pi, po, sink, fp, 1, K, 0ull, S);
+    // the neighbour is a fixed distance before the point
+    PoRecompute po(V.p, V.p - (isv ? V.NI : 1), S, depthu, K, c0);
+    UvSink<PoRecompute> sink{uu1, S, ub, pr, &po, 0ull, dpu1};
+    walk_core<METHOD, 1, PD, MIXED, false, true, false>(K, zx, pi, po, sink, fp, 1, K, 0ull, S, 0,
+                                                        c0);
   } else {
     PoSum po{dcol};
-    UvSink<PoSum> sink{uu, S, ub, pr, &po};
-    walk_core<METHOD, 1, PD, MIXED, false, true>(K, zx, pi, po, sink, fp, 1, K, 0ull, S);
+    UvSink<PoSum> sink{uu1, S, ub, pr, &po};
+    walk_core<METHOD, 1, PD, MIXED, false, true, false>(K, zx, pi, po, sink, fp, 1, K, 0ull, S, 0,
+                                                        c0);
 #pragma unroll 2
     for (int k = 1; k <= K; k++) dpu[(int64_t)(k - 1) * S] = dcol(k);
   }

@@ -241,8 +241,9 @@ int hycom_hybgen_set_kernel_path(int path);
 /* Variants of the streaming kernels (measurement and tuning; no reference
  * counterpart; results are bitwise the same for every value).  knob 0:
  * p-column remap variant, only 3 is built (a wave per pair of fields, 2
- * levels loaded ahead, new interfaces staged in LDS); knob 1: levels loaded ahead
- * by the u/v walk, 0, 2 or 4 (the default); knob 2: the u/v walk's new
+ * levels loaded ahead, new interfaces staged in LDS); knob 1: look-ahead of the u/v
+ * walk, 0, 2 or 4 (the default: the words of every layer loaded one layer
+ * before their use); knob 2: the u/v walk's new
  * thicknesses kept in LDS (0) or formed again from p as the walk needs them
  * (1, the default, no LDS); knob 3: the regrid's window loaded one
  * iteration ahead (1, the default) or not (0); knob 4: the u/v phase on a
@@ -253,11 +254,13 @@ int hycom_hybgen_tune(int knob, int value);
 /* Measurement hooks (no reference counterpart; the reference's only timer
  * is xctmr 49 around the whole call, mod_hycom.F90:2648-2653).  While
  * enabled, every hycom_hybgen_device() call records HIP events around its
- * phases on its stream: 0 column kernel (hybgenaj), 1 p halo, 2 u/v kernel
- * (dpudpv + hybgenbj), 3 Robert-Asselin kernel (hybgencj), 4 second halo,
+ * phases on its stream: 0 column kernels (hybgenaj, the p halo between them
+ * included), 1 p halo, 2 u/v kernel (dpudpv + hybgenbj) and the left-over
+ * columns and points, 3 Robert-Asselin kernel (hybgencj), 4 second halo,
  * 5 second u/v kernel; within phase 0 of the streaming kernels, 6 the
  * regrid kernel alone and 7 the p-column remap kernel alone (without its
- * fallback columns).  _read waits for the recorded calls, returns the
+ * fallback columns).  A small domain's remap and u/v kernels share a launch
+ * while this is off, and have one each while it is on.  _read waits for the recorded calls, returns the
  * summed milliseconds and call counts per phase, and forgets them. */
 int hycom_hybgen_timing(int enable);
 int hycom_hybgen_timing_read(double* ms_sum, int32_t* count, int nphase);
