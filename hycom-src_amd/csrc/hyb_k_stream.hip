@@ -56,6 +56,16 @@ k_regrid_a(KParams P, View V, Scratch W, int n) {
   regrid_stream<1>(P, V, W, i, j, n);
 }
 
+// first pass of the Robert-Asselin branch
+__global__ void __launch_bounds__(kWave) k_ra_pre(KParams P, View V, Scratch W, int m, int n) {
+  const int j = blockIdx.y + 1;
+  const int i = i_aligned0(V, j) + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 1 || i > P.ii) return;
+  const int64_t c0 = ij_of(V, i, j);
+  if (V.ip[c0] == 0) return;
+  W.kp[c0] = ra_pre(P, V, W, i, j, m, n);
+}
+
 bool stream_path_ok(const KParams& P) { return P.nhybrd == P.kk; }
 
 int uv_method_of(const KParams& P) { return uv_method(P); }
@@ -142,6 +152,8 @@ hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& 
   if (raflag) {
     {
       PhaseMark pm(T, s, 3);
+      dim3 gw((P.ii + kAlignPad + kWave - 1) / kWave, P.jj);
+      hipLaunchKernelGGL(k_ra_pre, gw, dim3(kWave), 0, s, P, V, W, m, n);
       switch (P.hybmap) {
         case 0: launch_ra_stream_m0(P, V, W, m, n, s); break;
         case 1: launch_ra_stream_m1(P, V, W, m, n, s); break;

@@ -2113,75 +2113,81 @@ HYB_HDI void remap_pair(const KParams& P, const View& V, const Scratch& W, int64
     remap_walk<METHOD, 1, PD, FAST, false>(P, V, c0, n, g0, K, zx, pres, kp, lcm, po);
 }
 
-// the last RA walk, over r < NF fields (r = 0: none)
+// RA walk of NW fields of level m from field g0 on: in place, or (staged)
+// into the workspace W.ras, from its field `slot` on, and over the fields once
+// the walk has read them (a walk of T alone leaves th3d to ra_post)
 template <int METHOD, int NW, int PD, class PO>
 HYB_HDI void ra_walk(const KParams& P, const View& V, const Scratch& W, int64_t c0, int m, int g0,
-                     int K, double zx, const PiRa& pi, uint64_t lcm, PO& po, bool staged) {
-  if (!staged) {
-    remap_walk_pi<METHOD, NW, PD, false, false>(P, V, c0, m, g0, K, zx, pi, K, lcm, po, K);
-    return;
-  }
-  // the outputs go to the workspace, then over the fields once the walk has
-  // read every level
+                     uint64_t lcm, PO& po, bool staged, int slot = 0) {
+  const int K = P.kk;
   const int64_t S = V.NIJ;
+  double* fp[NW];
   double* dst[NW];
-#pragma unroll
-  for (int f = 0; f < NW; f++) dst[f] = W.ras + (int64_t)f * K * S;
-  remap_walk_pi<METHOD, NW, PD, false, false>(P, V, c0, m, g0, K, zx, pi, K, lcm, po, K, dst);
 #pragma unroll
   for (int f = 0; f < NW; f++) {
     const int g = g0 + f;
-    double* fp = (g == 0) ? V.temp + c0 + lev4(V, 1, m)
-               : (g == 1) ? V.saln + c0 + lev4(V, 1, m)
-                          : V.tracer + c0 + levt(V, 1, m, g - 1);
-    stage_column(fp, 0, dst[f] + c0, S, K, S);
+    fp[f] = (g == 0) ? V.temp + lev4(V, 1, m)
+          : (g == 1) ? V.saln + lev4(V, 1, m)
+                     : V.tracer + levt(V, 1, m, g - 1);
+    dst[f] = staged ? W.ras + (int64_t)(slot + f) * K * S : fp[f];
+  }
+  const PiRa pi{W.pres, V.dp + lev4(V, 1, m), S};
+  const double zx = W.pres[(int64_t)K * S + c0];
+  remap_walk_pi<METHOD, NW, PD, false, false>(P, V, c0, m, g0, K, zx, pi, K, lcm, po, K, dst);
+  if (staged) {
+#pragma unroll
+    for (int f = 0; f < NW; f++) stage_column(fp[f] + c0, 0, dst[f] + c0, S, K, S);
   }
 }
-
-template <int METHOD, int R, int PD, class PO>
-HYB_HDI void ra_rest(const KParams& P, const View& V, const Scratch& W, int64_t c0, int m,
-                     int g0, int r, int K, double zx, const PiRa& pi, uint64_t lcm, PO& po,
-                     bool staged) {
-  if constexpr (R >= 1) {
-    if (r == R)
-      ra_walk<METHOD, R, PD>(P, V, W, c0, m, g0, K, zx, pi, lcm, po, staged);
-    else
-      ra_rest<METHOD, R - 1, PD>(P, V, W, c0, m, g0, r, K, zx, pi, lcm, po, staged);
-  }
+// pair q of the fields of level m
+template <int METHOD, int PD, class PO>
+HYB_HDI void ra_pair(const KParams& P, const View& V, const Scratch& W, int64_t c0, int m, int q,
+                     PO& po, bool staged) {
+  const int g0 = 2 * q, r = 2 + P.ntracr - g0;
+  const uint64_t lcm = W.lcm[c0];
+  if (r >= 2)
+    ra_walk<METHOD, 2, PD>(P, V, W, c0, m, g0, lcm, po, staged);
+  else if (r == 1)
+    ra_walk<METHOD, 1, PD>(P, V, W, c0, m, g0, lcm, po, staged);
 }
 
 // ---------------------------------------------------------------------
-// The Robert-Asselin branch of one p-column on the streaming design
-// (hybgencj, hybgen.F90:1909-2274), after hybgenaj has left the level-n
-// interfaces in p.  One pass over the column forms, without writing any
-// field:
+// The Robert-Asselin branch on the streaming design (hybgencj,
+// hybgen.F90:1909-2274), after hybgenaj has left the level-n interfaces in p
+// (the running sums of dp(n)).  ra_pre is its first pass over a column:
 //   * dp0ij and dp0cum from the level-n p (1931-1960) and the fixed layers
 //     from topiso (1962-1970);
 //   * the old level-m interfaces, running sums of dp(m), into the
 //     workspace;
 //   * the filtered thicknesses dp(m)+0.5*ra2fac*(dpo(n)+dp(n)-2*dpo(m))
-//     (2024-2032) and their running sums, the new interfaces, into the
-//     lane's LDS column (levels 2..K; 1 and K+1 in registers);
-//   * the PCM mask (2034-2046);
+//     (2024-2032) and their running sums, the new interfaces, into p, a
+//     level behind the level-n ones it reads there;
+//   * the PCM mask (2034-2046), into the workspace;
 //   * the in-place test of the walks (regrid_stream's) and the range test
 //     of the fast quotients.
-// A column that fails the range test returns false untouched, for
-// column_ra.  Otherwise T, S (with th3d) and the tracers of level m are
-// remapped by walk_core, with the old thicknesses dp(m) as stored (PiRa), no
-// massless fill, and the new grid's K layers (KO = K: its bottom need not
-// be the old one, and the column range covers every old level): in place,
-// or, where an output would overwrite a level the walk has not read (the
-// filtered bottom above the old one with massless layers below, for one),
-// into the workspace W.ras and then over the fields.  Then dp(m) is written
-// and p takes the level-m interfaces (2032).
+// The column's word in W.kp is kUnsafe where the range test fails (p is put
+// back, and the column left to column_ra), kStaged where an output would
+// overwrite a level the walk has not read (the filtered bottom above the old
+// one with massless layers below, for one), else 0.  Then T, S (with th3d)
+// and the tracers of level m are remapped by walk_core (ra_pair), with the
+// old thicknesses dp(m) as stored (PiRa), no massless fill, and the new
+// grid's K layers (KO = K: its bottom need not be the old one, and the column
+// range covers every old level): in place, or, where kStaged, through W.ras.
+// Last, dp(m) takes the filtered thicknesses (ra_post, 2032).
 // ---------------------------------------------------------------------
-template <int METHOD, int NF, int PD>
-HYB_HDI bool ra_stream(const KParams& P, const View& V, const Scratch& W, int i, int j, int m,
-                       int n, double* row, int ld) {
+constexpr int32_t kStaged = 1 << 17;
+
+HYB_HD double ra_thk(const KParams& P, double dold, double dnew, double dmid) {
+  const double qr = 0.5 * P.ra2fac * (dold + dnew - 2.0 * dmid);
+  return dmid + qr;
+}
+
+HYB_HDI int32_t ra_pre(const KParams& P, const View& V, const Scratch& W, int i, int j, int m,
+                       int n) {
   const int K = P.kk;
   const int64_t c0 = ij_of(V, i, j);
   const int64_t S = V.NIJ;
-  double* dpm = V.dp + c0 + lev4(V, 1, m);
+  const double* dpm = V.dp + c0 + lev4(V, 1, m);
   const double* dpn = V.dp + c0 + lev4(V, 1, n);
   const double* dpon = V.dpo + c0 + lev4(V, 1, n);
   const double* dpom = V.dpo + c0 + lev4(V, 1, m);
@@ -2217,9 +2223,7 @@ HYB_HDI bool ra_stream(const KParams& P, const View& V, const Scratch& W, int i,
       cum = cum + dp0;
     }
     const double prn = pr + dmk;
-    const double qr = 0.5 * P.ra2fac * (dold + dnew - 2.0 * dmid);
-    const double dk = dmid + qr;
-    const double psn = ps + dk;
+    const double psn = ps + ra_thk(P, dold, dnew, dmid);
     if (P.isopcm) {
       const bool v = !fixed && (dmk <= dpthin || dabs(thk - tak) < P.hybiso);
       if (v) lcm |= 1ull << (k - 1);
@@ -2233,18 +2237,18 @@ HYB_HDI bool ra_stream(const KParams& P, const View& V, const Scratch& W, int i,
       have = true;
     }
     pres[(int64_t)k * S] = prn;
+    pg[(int64_t)k * S] = psn;
     if (prn > pr) zlast = pr;
-    if (k <= K - 1) row[(int64_t)(k - 1) * ld] = psn;  // prsf(k+1) for k+1 in 2..K
     q0 = q1;
     q1 = pr;
     pr = prn;
     ps = psn;
   };
   {
-    // batches of 8 levels, the next batch loaded before the current one is
-    // used (indices clamped into the column; values beyond it unused);
-    // p(k) of level n is read here, before any of p is rewritten
-    constexpr int B = 8;
+    // batches of 4 levels, the next batch loaded before the current one is
+    // used (indices clamped into the column; values beyond it unused).  p(k)
+    // of level n is read at least a batch before p(k) is rewritten.
+    constexpr int B = 4;
     double a0[B], a1[B], a2[B], a3[B], a4[B], a5[B], a6[B];
     auto load = [&](int k0, double* x0, double* x1, double* x2, double* x3, double* x4,
                     double* x5, double* x6) {
@@ -2280,32 +2284,56 @@ HYB_HDI bool ra_stream(const KParams& P, const View& V, const Scratch& W, int i,
       }
     }
   }
-  const double zx = pr;  // pres(kk+1)
   // An output ending above zlast may overwrite a level the walk reads
   // later.  One ending below it ends in the deepest layer, which reaches the
   // bottom: the walk has folded every unread level into the column range at
   // the top of that layer (walk_core), every later output ends there too,
   // and nothing more is read.  (With the interfaces in order, tame.)
   const bool staged = have && cand <= zlast;
-  if (!tame || (staged && !W.ras)) return false;
-  StagedInterfaces po{row, ld, K + 1, 0.0, ps};
-  PiRa pi{W.pres, V.dp + lev4(V, 1, m), S};
-  const int nfields = 2 + P.ntracr;
-  int g0 = 0;
-  for (; g0 + NF <= nfields; g0 += NF)
-    ra_walk<METHOD, NF, PD>(P, V, W, c0, m, g0, K, zx, pi, lcm, po, staged);
-  ra_rest<METHOD, NF - 1, PD>(P, V, W, c0, m, g0, nfields - g0, K, zx, pi, lcm, po, staged);
-  // 2024-2032: dp(m) and the level-m interfaces
-  double sum = 0.0;
-#pragma unroll 4
+  W.lcm[c0] = lcm;
+  if (tame && !(staged && !W.ras)) return staged ? kStaged : 0;
+  double sum = 0.0;  // the level-n interfaces again
   for (int k = 1; k <= K; k++) {
-    const double qr = 0.5 * P.ra2fac * (dpon[(int64_t)(k - 1) * S] + dpn[(int64_t)(k - 1) * S] -
-                                        2.0 * dpom[(int64_t)(k - 1) * S]);
-    const double dk = dpom[(int64_t)(k - 1) * S] + qr;
-    dpm[(int64_t)(k - 1) * S] = dk;
-    sum = sum + dk;
+    sum = sum + dpn[(int64_t)(k - 1) * S];
     pg[(int64_t)k * S] = sum;
   }
+  return kUnsafe;
+}
+
+// dp(m) of levels k0, k0+st, ... (2024-2032), and th3d where T and S went
+// through the workspace apart
+HYB_HDI void ra_post(const KParams& P, const View& V, int64_t c0, int m, int n, int k0, int st,
+                     bool density) {
+  const int64_t S = V.NIJ;
+  double* dpm = V.dp + c0 + lev4(V, 1, m);
+  const double* dpn = V.dp + c0 + lev4(V, 1, n);
+  const double* dpon = V.dpo + c0 + lev4(V, 1, n);
+  const double* dpom = V.dpo + c0 + lev4(V, 1, m);
+#pragma unroll 4
+  for (int k = k0; k <= P.kk; k += st) {
+    const int64_t o = (int64_t)(k - 1) * S;
+    dpm[o] = ra_thk(P, dpon[o], dpn[o], dpom[o]);
+  }
+  if (density) {
+    for (int k = k0; k <= P.kk; k += st) {
+      const int64_t o = c0 + lev4(V, k, m);
+      V.th3d[o] = sig(V.temp[o], V.saln[o]) - P.thbase;
+    }
+  }
+}
+
+// the whole branch of one column, one lane (the device runs ra_pre and the
+// walks as two kernels)
+template <int METHOD, int NF, int PD>
+HYB_HDI bool ra_stream(const KParams& P, const View& V, const Scratch& W, int i, int j, int m,
+                       int n, double* row, int ld) {
+  const int64_t c0 = ij_of(V, i, j);
+  const int32_t st = ra_pre(P, V, W, i, j, m, n);
+  if (st & kUnsafe) return false;
+  StagedInterfaces po = stage_interfaces(row, ld, V.p + c0, V.NIJ, P.kk);
+  for (int q = 0; q < field_pairs(P); q++)
+    ra_pair<METHOD, PD>(P, V, W, c0, m, q, po, (st & kStaged) != 0);
+  ra_post(P, V, c0, m, n, 1, 1, false);
   return true;
 }
 
