@@ -136,8 +136,11 @@ void batch_layout(const KParams* hP, int nd, BatchLaunch& L, std::vector<int32_t
       return (int64_t)P.jj * ((P.ii + kAlignPad + cols - 1) / cols);
     };
   };
-  auto uvblocks = [](const KParams& P) {
-    return 2 * (int64_t)P.jj * ((P.ii + kAlignPad + 63) / 64);
+  // u, v (and p) points: `of` times the 64-wide row blocks
+  auto blocks64 = [](int of) {
+    return [of](const KParams& P) {
+      return of * (int64_t)P.jj * ((P.ii + kAlignPad + 63) / 64);
+    };
   };
   std::vector<int> all(nd);
   for (int d = 0; d < nd; d++) all[d] = d;
@@ -147,23 +150,27 @@ void batch_layout(const KParams* hP, int nd, BatchLaunch& L, std::vector<int32_t
   L.nremap = 0;
   for (int key = 0; key < kMaxGroups; key++) {
     std::vector<int> ds;
+    int pairs = 0;
     for (int d = 0; d < nd; d++)
-      if (hP[d].hybmap + 4 * hP[d].precision == key) ds.push_back(d);
-    if (!ds.empty()) group(ds, rows(L.remap_cols), key, &L.remap[L.nremap++]);
+      if (hP[d].hybmap + 4 * hP[d].precision == key) {
+        ds.push_back(d);
+        const int p = (2 + hP[d].ntracr + 1) / 2;
+        pairs = p > pairs ? p : pairs;
+      }
+    if (ds.empty()) continue;
+    L.remap[L.nremap].pairs = pairs;
+    group(ds, rows(64), key, &L.remap[L.nremap++]);
   }
-  group(all, rows(64), 0, &L.rows64);
-  group(all, [](const KParams& P) { return (int64_t)P.kk * ((P.ii + 255) / 256); }, 0,
-        &L.halo_j);
-  group(all, [](const KParams& P) { return (int64_t)P.kk * ((P.jj + 2 + 255) / 256); }, 0,
-        &L.halo_i);
+  group(all, [](const KParams& P) { return (int64_t)P.kk * ((P.ii + P.jj + 2 + 255) / 256); }, 0,
+        &L.halo);
   L.nuv = 0;
   for (int key = 0; key < kMaxGroups; key++) {
     std::vector<int> ds;
     for (int d = 0; d < nd; d++)
       if (uv_method_of(hP[d]) + 4 * hP[d].precision == key) ds.push_back(d);
-    if (!ds.empty()) group(ds, uvblocks, key, &L.uv[L.nuv++]);
+    if (!ds.empty()) group(ds, blocks64(2), key, &L.uv[L.nuv++]);
   }
-  group(all, uvblocks, 0, &L.uvall);
+  group(all, blocks64(3), 0, &L.rest);
 }
 
 void batch_bind(BatchLaunch& L, const int32_t* dI) {
@@ -173,11 +180,9 @@ void batch_bind(BatchLaunch& L, const int32_t* dI) {
   };
   fix(L.regrid);
   for (int q = 0; q < L.nremap; q++) fix(L.remap[q]);
-  fix(L.rows64);
-  fix(L.halo_j);
-  fix(L.halo_i);
+  fix(L.halo);
   for (int q = 0; q < L.nuv; q++) fix(L.uv[q]);
-  fix(L.uvall);
+  fix(L.rest);
 }
 
 }  // namespace hyb
@@ -610,151 +615,102 @@ int hycom_hybgen_record_decisions(int32_t* fixlay_dev, int32_t* kp_dev) {
 // ---------------------------------------------------------------------
 namespace {
 
+// A domain set prepared for the batch kernels: the descriptors (parameters,
+// field views, workspaces and block layouts) of its launches in one device
+// buffer.  The last kPlans sets are kept, keyed by the bytes of everything
+// the descriptors hold, so callers that alternate between a few sets do not
+// prepare them again; preparing one is a copy of some kilobytes on a stream of
+// its own and does not wait for running batches.  (One set kept, with its
+// arrays freed and allocated, and a graph captured, at every change: 24
+// domains, three sets in turn, 4.9 ms a call of which 0.4 ms was the change.)
 struct BatchPlan {
-  std::vector<unsigned char> key;  // the KParams and View of every domain
+  std::vector<unsigned char> key;  // KParams, View and Scratch of every domain
   int ndom = 0;
-  KParams* dP = nullptr;
-  View* dV = nullptr;
-  Scratch* dW = nullptr;
-  int32_t* dI = nullptr;
-  size_t nI = 0;
+  unsigned char* dev = nullptr;
+  size_t cap = 0;
   BatchDevice B{};
   BatchLaunch L{};
-  hipStream_t cap = nullptr;
-  hipGraph_t graph[2] = {nullptr, nullptr};
-  hipGraphExec_t exec[2] = {nullptr, nullptr};  // per time level n
-  // online autotuning: first the remap workgroups (columns, staged
-  // interface levels) with 256-column regrid workgroups, then the regrid
-  // widths with the best remap candidate
-  struct Cand {
-    int rc, ns, gc;  // remap columns, staged levels, regrid columns
-  };
-  std::vector<Cand> cands;
-  std::vector<float> ms;  // best time of each candidate
-  int cand = 0;           // candidate measured by the pending events
-  int rep = 0;            // measurements of it so far
-  bool second = false;    // the regrid widths are being searched
+  // online autotuning of the regrid's workgroup width
+  std::vector<int> cands;  // columns per regrid workgroup
+  std::vector<float> ms;   // best time of each candidate
+  int cand = 0;            // candidate measured by the pending events
+  int rep = 0;             // measurements of it so far
   bool pending = false, tuned = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  hipEvent_t done = nullptr;  // after the last launch of this plan's graphs
+  hipEvent_t done = nullptr;  // after the last launch of this plan
+  hipStream_t last = nullptr; // that launch's stream
   bool launched = false;
+  int64_t used = 0;
   std::vector<KParams> hP;
   std::vector<View> hV;
+  std::vector<Scratch> hW;
 };
+constexpr int kPlans = 4;
 std::mutex g_batch_mu;
-BatchPlan g_plan;
+BatchPlan g_plans[64][kPlans];  // per device
+BatchPlan g_no_plan;
+BatchPlan* g_plan = &g_no_plan;  // the last batch's
+hipStream_t g_batch_up[64] = {};
+int64_t g_batch_clock = 0;
 bool g_batch_autotune = true;
 
-void plan_drop_graphs(BatchPlan& b) {
-  for (int q = 0; q < 2; q++) {
-    if (b.exec[q]) (void)hipGraphExecDestroy(b.exec[q]);
-    if (b.graph[q]) (void)hipGraphDestroy(b.graph[q]);
-    b.exec[q] = nullptr;
-    b.graph[q] = nullptr;
-  }
-}
-
-// waits for the last launch of the plan's graphs before its arrays change
+// waits for the last launch of the plan before its buffer changes
 int plan_quiesce(BatchPlan& b) {
   if (b.launched) HIPCHK(hipEventSynchronize(b.done));
   b.launched = false;
   return 0;
 }
 
-void plan_free(BatchPlan& b) {
-  plan_drop_graphs(b);
-  if (b.dP) (void)hipFree(b.dP);
-  if (b.dV) (void)hipFree(b.dV);
-  if (b.dW) (void)hipFree(b.dW);
-  if (b.dI) (void)hipFree(b.dI);
-  b.dP = nullptr;
-  b.dV = nullptr;
-  b.dW = nullptr;
-  b.dI = nullptr;
-  b.nI = 0;
-  b.key.clear();
-}
-
-// block layouts of every launch for the current widths
-int plan_layout(BatchPlan& b) {
+// the descriptors for the current widths, copied and in place on return
+int plan_layout(BatchPlan& b, int dev) {
   if (int rc = plan_quiesce(b)) return rc;
   std::vector<int32_t> I;
   batch_layout(b.hP.data(), b.ndom, b.L, I);
-  if (I.size() > b.nI) {
-    if (b.dI) (void)hipFree(b.dI);
-    b.dI = nullptr;
-    HIPCHK(hipMalloc(&b.dI, sizeof(int32_t) * I.size()));
-    b.nI = I.size();
+  auto up = [](size_t x) { return (x + 255) & ~size_t(255); };
+  const size_t oV = up(sizeof(KParams) * b.ndom), oW = oV + up(sizeof(View) * b.ndom);
+  const size_t oI = oW + up(sizeof(Scratch) * b.ndom), n = oI + sizeof(int32_t) * I.size();
+  if (n > b.cap) {
+    if (b.dev) (void)hipFree(b.dev);
+    b.dev = nullptr;
+    b.cap = 0;
+    HIPCHK(hipMalloc(&b.dev, 2 * n));
+    b.cap = 2 * n;
   }
-  HIPCHK(hipMemcpy(b.dI, I.data(), sizeof(int32_t) * I.size(), hipMemcpyHostToDevice));
-  batch_bind(b.L, b.dI);
-  plan_drop_graphs(b);
+  std::vector<unsigned char> h(n);
+  memcpy(h.data(), b.hP.data(), sizeof(KParams) * b.ndom);
+  memcpy(h.data() + oV, b.hV.data(), sizeof(View) * b.ndom);
+  memcpy(h.data() + oW, b.hW.data(), sizeof(Scratch) * b.ndom);
+  memcpy(h.data() + oI, I.data(), sizeof(int32_t) * I.size());
+  hipStream_t& us = g_batch_up[dev];
+  if (!us) HIPCHK(hipStreamCreateWithFlags(&us, hipStreamNonBlocking));
+  HIPCHK(hipMemcpyAsync(b.dev, h.data(), n, hipMemcpyHostToDevice, us));
+  HIPCHK(hipStreamSynchronize(us));
+  b.B = BatchDevice{(const KParams*)b.dev, (const View*)(b.dev + oV), (const Scratch*)(b.dev + oW)};
+  batch_bind(b.L, (const int32_t*)(b.dev + oI));
   return 0;
 }
 
-int plan_graph(BatchPlan& b, int n) {
-  const int q = n - 1;
-  if (b.exec[q]) return 0;
-  if (!b.cap) HIPCHK(hipStreamCreateWithFlags(&b.cap, hipStreamNonBlocking));
-  HIPCHK(hipStreamBeginCapture(b.cap, hipStreamCaptureModeThreadLocal));
-  hipError_t e = launch_batch(b.B, b.L, n, b.cap);
-  hipGraph_t g = nullptr;
-  hipError_t e2 = hipStreamEndCapture(b.cap, &g);
-  HIPCHK(e);
-  HIPCHK(e2);
-  b.graph[q] = g;
-  HIPCHK(hipGraphInstantiate(&b.exec[q], g, nullptr, nullptr, 0));
-  return 0;
-}
-
-int plan_build(BatchPlan& b, const hyb_domain* D, int ndom, std::vector<unsigned char>& key) {
+int plan_build(BatchPlan& b, int dev, std::vector<unsigned char>& key, std::vector<KParams>& hP,
+               std::vector<View>& hV, std::vector<Scratch>& hW) {
   if (int rc = plan_quiesce(b)) return rc;
-  plan_free(b);
-  b.ndom = ndom;
-  b.hP.resize(ndom);
-  b.hV.resize(ndom);
-  std::vector<Scratch> hW(ndom);
-  for (int d = 0; d < ndom; d++) {
-    b.hP[d] = kparams_of(D[d].P);
-    b.hV[d] = view_of(D[d].P, D[d].F);
-    int rc = workspace_for(D[d].F->p, b.hV[d].NIJ, D[d].P->kdm, &hW[d]);
-    if (rc) return rc;
-  }
-  HIPCHK(hipMalloc(&b.dP, sizeof(KParams) * ndom));
-  HIPCHK(hipMalloc(&b.dV, sizeof(View) * ndom));
-  HIPCHK(hipMalloc(&b.dW, sizeof(Scratch) * ndom));
-  HIPCHK(hipMemcpy(b.dP, b.hP.data(), sizeof(KParams) * ndom, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(b.dV, b.hV.data(), sizeof(View) * ndom, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(b.dW, hW.data(), sizeof(Scratch) * ndom, hipMemcpyHostToDevice));
-  b.B = BatchDevice{b.dP, b.dV, b.dW};
-  int kmax = 0;
-  for (int d = 0; d < ndom; d++) kmax = b.hP[d].kk > kmax ? b.hP[d].kk : kmax;
-  // remap candidates: a workgroup stages ns interface levels of each of
-  // its columns in LDS (ns x cols doubles, at most 64 KB): all kmax-1, or
-  // 24 or 12 with the deeper levels read from p as the walk reaches them
-  b.cands.clear();
-  const int lvl = kmax > 1 ? kmax - 1 : 1;
-  for (int rc : {64, 128, 256})
-    for (int ns : {lvl, 24, 12}) {
-      if (ns != lvl && ns >= lvl) continue;  // a split stages fewer levels than all
-      if (sizeof(double) * ns * rc <= 65536) b.cands.push_back({rc, ns, 256});
-    }
+  b.key.clear();  // until the plan is whole again
+  b.ndom = (int)hP.size();
+  b.hP.swap(hP);
+  b.hV.swap(hV);
+  b.hW.swap(hW);
+  b.cands = {256, 128, 64};
   b.ms.assign(b.cands.size(), -1.0f);
   b.cand = 0;
   b.rep = 0;
-  b.second = false;
   b.pending = false;
   b.tuned = !g_batch_autotune;
-  // first candidate (and the untuned widths): 64-column remaps staging every
-  // level, 256-column regrid
-  b.L.remap_cols = b.cands[0].rc;
-  b.L.remap_stage = b.cands[0].ns;
-  b.L.regrid_cols = b.cands[0].gc;
+  b.L.regrid_cols = b.cands[0];  // also the untuned width
   if (!b.ev0) HIPCHK(hipEventCreate(&b.ev0));
   if (!b.ev1) HIPCHK(hipEventCreate(&b.ev1));
   if (!b.done) HIPCHK(hipEventCreateWithFlags(&b.done, hipEventDisableTiming));
-  b.key = key;
-  return plan_layout(b);
+  if (int rc = plan_layout(b, dev)) return rc;
+  b.key.swap(key);
+  return 0;
 }
 
 }  // namespace
@@ -771,16 +727,9 @@ int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream
       if (D[e].F->p == D[d].F->p) return fail(HYB_EINVAL, "domains %d and %d share p", e, d);
   }
   if ((rc = device_ready())) return rc;
-  std::vector<unsigned char> key;
-  key.reserve(ndom * (sizeof(KParams) + sizeof(View)));
-  for (int d = 0; d < ndom; d++) {
-    KParams k = kparams_of(D[d].P);
-    View v = view_of(D[d].P, D[d].F);
-    const unsigned char* a = (const unsigned char*)&k;
-    key.insert(key.end(), a, a + sizeof k);
-    a = (const unsigned char*)&v;
-    key.insert(key.end(), a, a + sizeof v);
-  }
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64) return fail(HYB_EDEVICE, "device ordinal %d out of range", dev);
   for (int d = 0; d < ndom; d++)
     if (D[d].P->check_finite) {
       const KParams K = kparams_of(D[d].P);
@@ -788,9 +737,36 @@ int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream
       if ((rc = scan_finite(K, V, n, (hipStream_t)stream))) return rc;
     }
   std::lock_guard<std::mutex> lk(g_batch_mu);
-  BatchPlan& b = g_plan;
-  if (b.key != key || b.ndom != ndom) {
-    if ((rc = plan_build(b, D, ndom, key))) return rc;
+  std::vector<KParams> hP(ndom);
+  std::vector<View> hV(ndom);
+  std::vector<Scratch> hW(ndom);
+  std::vector<unsigned char> key;
+  key.reserve(ndom * (sizeof(KParams) + sizeof(View) + sizeof(Scratch)));
+  auto add = [&](const void* a, size_t bytes) {
+    key.insert(key.end(), (const unsigned char*)a, (const unsigned char*)a + bytes);
+  };
+  for (int d = 0; d < ndom; d++) {
+    hP[d] = kparams_of(D[d].P);
+    hV[d] = view_of(D[d].P, D[d].F);
+    memset(&hW[d], 0, sizeof(Scratch));
+    if ((rc = workspace_for(D[d].F->p, hV[d].NIJ, D[d].P->kdm, &hW[d]))) return rc;
+    add(&hP[d], sizeof(KParams));
+    add(&hV[d], sizeof(View));
+    add(&hW[d], sizeof(Scratch));
+  }
+  BatchPlan* slot = &g_plans[dev][0];
+  for (BatchPlan& q : g_plans[dev]) {
+    if (q.ndom == ndom && q.key == key) {
+      slot = &q;
+      break;
+    }
+    if (q.used < slot->used) slot = &q;  // else the one not used for longest
+  }
+  BatchPlan& b = *slot;
+  b.used = ++g_batch_clock;
+  g_plan = slot;
+  if (b.ndom != ndom || b.key != key) {
+    if ((rc = plan_build(b, dev, key, hP, hV, hW))) return rc;
   }
   hipStream_t s = (hipStream_t)stream;
   // autotuning: read the pending measurement, move to the next candidate
@@ -800,43 +776,36 @@ int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream
     HIPCHK(hipEventElapsedTime(&t, b.ev0, b.ev1));
     b.ms[b.cand] = (b.rep == 0 || t < b.ms[b.cand]) ? t : b.ms[b.cand];
     b.pending = false;
-    // two launches per candidate: the first one also loads the graph
+    // two launches per candidate
     if (++b.rep == 2) {
       b.rep = 0;
       int next = ++b.cand;
       if (next >= (int)b.cands.size()) {
-        int best = 0;
+        next = 0;
         for (int q = 1; q < (int)b.cands.size(); q++)
-          if (b.ms[q] < b.ms[best]) best = q;
-        next = best;
-        if (!b.second) {
-          // the regrid widths, with the best remap workgroup
-          b.second = true;
-          const BatchPlan::Cand w = b.cands[best];
-          for (int gc : {128, 64}) {
-            b.cands.push_back({w.rc, w.ns, gc});
-            b.ms.push_back(-1.0f);
-          }
-          next = b.cand;
-        } else {
-          b.tuned = true;
+          if (b.ms[q] < b.ms[next]) next = q;
+        b.tuned = true;
+      }
+      if (b.L.regrid_cols != b.cands[next]) {
+        b.L.regrid_cols = b.cands[next];
+        if ((rc = plan_layout(b, dev))) {
+          b.key.clear();  // prepared again by the next call
+          return rc;
         }
       }
-      b.L.remap_cols = b.cands[next].rc;
-      b.L.remap_stage = b.cands[next].ns;
-      b.L.regrid_cols = b.cands[next].gc;
-      if ((rc = plan_layout(b))) return rc;
     }
   }
-  if ((rc = plan_graph(b, n))) return rc;
+  // one set on two streams: the second call's launches follow the first's
+  if (b.launched && b.last != s) HIPCHK(hipStreamWaitEvent(s, b.done, 0));
   const bool measure = !b.tuned;
   if (measure) HIPCHK(hipEventRecord(b.ev0, s));
-  HIPCHK(hipGraphLaunch(b.exec[n - 1], s));
+  HIPCHK(launch_batch(b.B, b.L, n, s));
   if (measure) {
     HIPCHK(hipEventRecord(b.ev1, s));
     b.pending = true;
   }
   HIPCHK(hipEventRecord(b.done, s));
+  b.last = s;
   b.launched = true;
   (void)m;
   return 0;
@@ -850,9 +819,9 @@ int hycom_hybgen_batch_autotune(int enable) {
 
 int hycom_hybgen_batch_config(int32_t* remap_cols, int32_t* regrid_cols, int32_t* tuned) {
   std::lock_guard<std::mutex> lk(g_batch_mu);
-  if (remap_cols) *remap_cols = g_plan.L.remap_cols;
-  if (regrid_cols) *regrid_cols = g_plan.L.regrid_cols;
-  if (tuned) *tuned = g_plan.tuned ? 1 : 0;
+  if (remap_cols) *remap_cols = g_plan->L.kmax > 0 ? 64 : 0;
+  if (regrid_cols) *regrid_cols = g_plan->L.regrid_cols;
+  if (tuned) *tuned = g_plan->tuned ? 1 : 0;
   return 0;
 }
 
@@ -860,20 +829,20 @@ int hycom_hybgen_batch_tuning(int32_t* remap_cols, int32_t* staged_levels,
                               int32_t* regrid_cols, float* ms, int cap) {
   std::lock_guard<std::mutex> lk(g_batch_mu);
   if (cap < 0) return fail(HYB_EINVAL, "cap %d", cap);
-  const int nc = (int)g_plan.cands.size();
+  const int nc = (int)g_plan->cands.size();
   for (int q = 0; q < nc && q < cap; q++) {
-    if (remap_cols) remap_cols[q] = g_plan.cands[q].rc;
-    if (staged_levels) staged_levels[q] = g_plan.cands[q].ns;
-    if (regrid_cols) regrid_cols[q] = g_plan.cands[q].gc;
-    if (ms) ms[q] = g_plan.ms[q];
+    if (remap_cols) remap_cols[q] = 64;
+    if (staged_levels) staged_levels[q] = batch_stage_levels(g_plan->L);
+    if (regrid_cols) regrid_cols[q] = g_plan->cands[q];
+    if (ms) ms[q] = g_plan->ms[q];
   }
   return nc;
 }
 
 int hycom_hybgen_batch_staged_levels(int32_t* levels, int32_t* kmax) {
   std::lock_guard<std::mutex> lk(g_batch_mu);
-  if (levels) *levels = g_plan.L.kmax > 0 ? batch_stage_levels(g_plan.L) : 0;
-  if (kmax) *kmax = g_plan.L.kmax;
+  if (levels) *levels = g_plan->L.kmax > 0 ? batch_stage_levels(g_plan->L) : 0;
+  if (kmax) *kmax = g_plan->L.kmax;
   return 0;
 }
 

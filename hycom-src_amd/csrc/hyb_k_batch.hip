@@ -98,69 +98,47 @@ kb_regrid(BatchDevice B, BatchGroup G, int n) {
   regrid_stream<1>(P, V, gscratch(B.W, r.d), i, r.j, n);
 }
 
-// CW columns per workgroup; each lane's LDS column has stride CW doubles
-// and holds ns levels of the new interfaces: all of them (SPLIT false), or
-// the upper ns with the rest read from p (the split costs the walk a few
-// registers and branches, so the whole column keeps its own instance)
-template <int METHOD, bool MIXED, int CW, bool SPLIT>
-__global__ void __launch_bounds__(CW) kb_remap(BatchDevice B, BatchGroup G, int n, int ns) {
+// The p-column remap: 64 columns by one wave per pair of fields (blockDim.y
+// waves, for the domain with the most fields of the group; a domain's other
+// waves only help to stage the new interfaces), as k_remap_s.  One wave
+// walking three fields at a time over 64 columns, against this: 24 domains of
+// 60-480 x 60-360 x 22/32/41 with 4 fields, 3.0 against 1.5 ms.
+template <int METHOD, bool MIXED>
+__global__ void __launch_bounds__(kWave * kRemapWaves) __attribute__((amdgpu_waves_per_eu(3)))
+kb_remap(BatchDevice B, BatchGroup G, int n) {
   extern __shared__ double lds[];
-  const RowPos r = row_pos(B, G, CW, blockIdx.x);
-  const KParams& P = B.P[r.d];
-  const View V = gview(B.V, r.d);
-  const Scratch W = gscratch(B.W, r.d);
-  const int i = r.i0 + threadIdx.x;
-  if (i < 1 || i > P.ii) return;
-  const int64_t c0 = ij_of(V, i, r.j);
-  const int32_t ipw = V.ip[c0], kpw = W.kp[c0];  // kp of a land column: read, not used
-  if ((ipw == 0) | ((kpw & kUnsafe) != 0)) return;
-  if (SPLIT) {
-    SplitInterfaces po = stage_split(lds + threadIdx.x, CW, V.p + c0, V.NIJ, P.kk, ns);
-    if (MIXED) remap_mixed<METHOD, 3, 2>(P, V, W, i, r.j, n, po);
-    else remap_stream<METHOD, 3, 2>(P, V, W, i, r.j, n, po);
-  } else {
-    StagedInterfaces po = stage_interfaces(lds + threadIdx.x, CW, V.p + c0, V.NIJ, P.kk);
-    if (MIXED) remap_mixed<METHOD, 3, 2>(P, V, W, i, r.j, n, po);
-    else remap_stream<METHOD, 3, 2>(P, V, W, i, r.j, n, po);
-  }
-}
-
-__global__ void __launch_bounds__(kWave) kb_remap_fb(BatchDevice B, BatchGroup G, int n) {
   const RowPos r = row_pos(B, G, kWave, blockIdx.x);
   const KParams& P = B.P[r.d];
   const View V = gview(B.V, r.d);
   const Scratch W = gscratch(B.W, r.d);
   const int i = r.i0 + threadIdx.x;
-  if (i < 1 || i > P.ii) return;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
   const int64_t c0 = ij_of(V, i, r.j);
-  if (V.ip[c0] == 0) return;
-  if (!(W.kp[c0] & kUnsafe)) return;
-  remap_fallback(P, V, W, i, r.j, n);
+  bool on = i >= 1 && i <= P.ii;
+  int32_t kpw = 0;
+  if (on) {
+    const int32_t ipw = V.ip[c0];  // kp of a land column: read, not used
+    kpw = W.kp[c0];
+    on = (ipw != 0) & ((kpw & kUnsafe) == 0);
+  }
+  double* row = lds + threadIdx.x;
+  StagedInterfaces po{row, kWave, P.kk + 1, 0.0, 0.0};
+  if (on) po = stage_interfaces_part(row, kWave, V.p + c0, V.NIJ, P.kk, w, blockDim.y);
+  __syncthreads();
+  if (!on) return;
+  remap_pair<METHOD, 2, MIXED>(P, V, W, c0, n, kpw, blockIdx.y * kRemapWaves + w, po);
 }
 
-// p halo of every domain, levels 2..kk+1: the j rows, then the i columns
-// (mod_xc_sm.h:1374-1424).  Blocks: kk per domain and 256-wide slice.
-__global__ void __launch_bounds__(kBlock) kb_halo_j(BatchDevice B, BatchGroup G) {
+// p halo of every domain, levels 2..kk+1 (mod_xc_sm.h:1374-1424).  Blocks:
+// kk per domain and 256-wide slice of the halo points.
+__global__ void __launch_bounds__(kBlock) kb_halo(BatchDevice B, BatchGroup G) {
   const int g = group_of(G.prefix, G.ndom, blockIdx.x);
   const int d = G.dom[g];
   const KParams& P = B.P[d];
   const int local = blockIdx.x - G.prefix[g];
-  const int nbi = (P.ii + kBlock - 1) / kBlock;
-  const int k = local / nbi + 2;
-  const int i = (local % nbi) * kBlock + threadIdx.x + 1;
-  if (i > P.ii) return;
-  p_halo_jrow(P, gview(B.V, d), i, k);
-}
-__global__ void __launch_bounds__(kBlock) kb_halo_i(BatchDevice B, BatchGroup G) {
-  const int g = group_of(G.prefix, G.ndom, blockIdx.x);
-  const int d = G.dom[g];
-  const KParams& P = B.P[d];
-  const int local = blockIdx.x - G.prefix[g];
-  const int nbj = (P.jj + 2 + kBlock - 1) / kBlock;
-  const int k = local / nbj + 2;
-  const int j = (local % nbj) * kBlock + threadIdx.x;
-  if (j > P.jj + 1) return;
-  p_halo_icol(P, gview(B.V, d), j, k);
+  const int nb = (P.ii + P.jj + 2 + kBlock - 1) / kBlock;
+  const int t = (local % nb) * kBlock + threadIdx.x;
+  if (t < P.ii + P.jj + 2) p_halo_point(P, gview(B.V, d), t, local / nb + 2);
 }
 
 // u- and v-points: the first half of a domain's blocks are u, then v
@@ -182,63 +160,52 @@ __global__ void __launch_bounds__(kWave) kb_uv(BatchDevice B, BatchGroup G, int 
   const int32_t* msk = isv ? V.iv : V.iu;
   if (msk[c0] == 0) return;
   LaneRow dcol{lds + threadIdx.x, kWave};  // unused: new thicknesses formed again from p
-  const bool ok = uv_stream<METHOD, 4, MIXED, true>(P, V, i, j, nl, isv, dcol);
+  const bool ok = uv_stream<METHOD, 1, MIXED, true>(P, V, i, j, nl, isv, dcol);
   gscratch(B.W, d).uvf[c0 + (isv ? V.NIJ : 0)] = ok ? 0 : 1;
 }
 
-__global__ void __launch_bounds__(kWave) kb_uv_fb(BatchDevice B, BatchGroup G, int nl) {
+// the columns and the u- and v-points left over: a third of a domain's
+// blocks each
+__global__ void __launch_bounds__(kWave) kb_fb(BatchDevice B, BatchGroup G, int n) {
   const int g = group_of(G.prefix, G.ndom, blockIdx.x);
   const int d = G.dom[g];
   const KParams& P = B.P[d];
   const View V = gview(B.V, d);
+  const Scratch W = gscratch(B.W, d);
   const int nbi = (P.ii + kAlignPad + kWave - 1) / kWave;
-  int local = blockIdx.x - G.prefix[g];
-  const bool isv = local >= P.jj * nbi;
-  if (isv) local -= P.jj * nbi;
-  const int j = local / nbi + 1;
-  const int i = i_aligned0(V, j) + (local % nbi) * kWave + threadIdx.x;
+  const int local = blockIdx.x - G.prefix[g];
+  const int z = local / (P.jj * nbi), rest = local % (P.jj * nbi);  // p, u, v
+  const int j = rest / nbi + 1;
+  const int i = i_aligned0(V, j) + (rest % nbi) * kWave + threadIdx.x;
   if (i < 1 || i > P.ii) return;
   const int64_t c0 = ij_of(V, i, j);
-  const int32_t* msk = isv ? V.iv : V.iu;
-  if (msk[c0] == 0) return;
-  if (gscratch(B.W, d).uvf[c0 + (isv ? V.NIJ : 0)] == 0) return;
-  point_c<64>(P, V, i, j, nl, isv);
-}
-
-template <int CW, bool SPLIT>
-static void remap_group_cw(const BatchDevice& B, const BatchGroup& G, int n, int ns,
-                           hipStream_t s) {
-  const dim3 grid(G.nblocks), blk(CW);
-  const size_t lds = sizeof(double) * ns * CW;
-  switch (G.key) {  // hybmap + 4 * precision
-    case 0: hipLaunchKernelGGL((kb_remap<0, false, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
-    case 1: hipLaunchKernelGGL((kb_remap<1, false, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
-    case 2: hipLaunchKernelGGL((kb_remap<2, false, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
-    case 3: hipLaunchKernelGGL((kb_remap<3, false, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
-    case 4: hipLaunchKernelGGL((kb_remap<0, true, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
-    case 5: hipLaunchKernelGGL((kb_remap<1, true, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
-    case 6: hipLaunchKernelGGL((kb_remap<2, true, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
-    default: hipLaunchKernelGGL((kb_remap<3, true, CW, SPLIT>), grid, blk, lds, s, B, G, n, ns); break;
+  if (z == 0) {
+    if (V.ip[c0] == 0) return;
+    if (!(W.kp[c0] & kUnsafe)) return;
+    remap_fallback(P, V, W, i, j, n);
+  } else {
+    const bool isv = z == 2;
+    if ((isv ? V.iv : V.iu)[c0] == 0) return;
+    if (W.uvf[c0 + (isv ? V.NIJ : 0)] == 0) return;
+    point_c<64>(P, V, i, j, n, isv);
   }
 }
 
-// the interface levels a remap workgroup stages per column: remap_stage
-// (0: all, kmax-1), at most kmax-1
-int batch_stage_levels(const BatchLaunch& L) {
-  const int all = lds_levels(L.kmax);
-  return (L.remap_stage > 0 && L.remap_stage < all) ? L.remap_stage : all;
-}
+// the interface levels a remap workgroup stages per column
+int batch_stage_levels(const BatchLaunch& L) { return lds_levels(L.kmax); }
 
-static void remap_group(const BatchDevice& B, const BatchGroup& G, int n, int ns, bool split,
-                        int cw, hipStream_t s) {
-  if (split) {
-    if (cw == 256) remap_group_cw<256, true>(B, G, n, ns, s);
-    else if (cw == 128) remap_group_cw<128, true>(B, G, n, ns, s);
-    else remap_group_cw<64, true>(B, G, n, ns, s);
-  } else {  // every level staged: at most 64 KB with 64 or 128 columns
-    if (cw == 256) remap_group_cw<256, false>(B, G, n, ns, s);
-    else if (cw == 128) remap_group_cw<128, false>(B, G, n, ns, s);
-    else remap_group_cw<64, false>(B, G, n, ns, s);
+static void remap_group(const BatchDevice& B, const BatchGroup& G, int n, int ns, hipStream_t s) {
+  const dim3 grid(G.nblocks, remap_blocks(G.pairs)), blk(kWave, remap_waves(G.pairs));
+  const size_t lds = sizeof(double) * ns * kWave;
+  switch (G.key) {  // hybmap + 4 * precision
+    case 0: hipLaunchKernelGGL((kb_remap<0, false>), grid, blk, lds, s, B, G, n); break;
+    case 1: hipLaunchKernelGGL((kb_remap<1, false>), grid, blk, lds, s, B, G, n); break;
+    case 2: hipLaunchKernelGGL((kb_remap<2, false>), grid, blk, lds, s, B, G, n); break;
+    case 3: hipLaunchKernelGGL((kb_remap<3, false>), grid, blk, lds, s, B, G, n); break;
+    case 4: hipLaunchKernelGGL((kb_remap<0, true>), grid, blk, lds, s, B, G, n); break;
+    case 5: hipLaunchKernelGGL((kb_remap<1, true>), grid, blk, lds, s, B, G, n); break;
+    case 6: hipLaunchKernelGGL((kb_remap<2, true>), grid, blk, lds, s, B, G, n); break;
+    default: hipLaunchKernelGGL((kb_remap<3, true>), grid, blk, lds, s, B, G, n); break;
   }
 }
 
@@ -265,18 +232,13 @@ hipError_t launch_batch(const BatchDevice& B, const BatchLaunch& L, int n, hipSt
     else
       hipLaunchKernelGGL(kb_regrid<64>, grid, dim3(64), 0, s, B, L.regrid, n);
   }
-  const int ns = batch_stage_levels(L);
-  const bool split = ns < lds_levels(L.kmax);
-  for (int q = 0; q < L.nremap; q++) remap_group(B, L.remap[q], n, ns, split, L.remap_cols, s);
-  if (L.rows64.nblocks > 0)
-    hipLaunchKernelGGL(kb_remap_fb, dim3(L.rows64.nblocks), dim3(kWave), 0, s, B, L.rows64, n);
-  if (L.halo_j.nblocks > 0)
-    hipLaunchKernelGGL(kb_halo_j, dim3(L.halo_j.nblocks), dim3(kBlock), 0, s, B, L.halo_j);
-  if (L.halo_i.nblocks > 0)
-    hipLaunchKernelGGL(kb_halo_i, dim3(L.halo_i.nblocks), dim3(kBlock), 0, s, B, L.halo_i);
+  if (L.halo.nblocks > 0)
+    hipLaunchKernelGGL(kb_halo, dim3(L.halo.nblocks), dim3(kBlock), 0, s, B, L.halo);
+  for (int q = 0; q < L.nremap; q++)
+    remap_group(B, L.remap[q], n, batch_stage_levels(L), s);
   for (int q = 0; q < L.nuv; q++) uv_group(B, L.uv[q], n, 0, s);
-  if (L.uvall.nblocks > 0)
-    hipLaunchKernelGGL(kb_uv_fb, dim3(L.uvall.nblocks), dim3(kWave), 0, s, B, L.uvall, n);
+  if (L.rest.nblocks > 0)
+    hipLaunchKernelGGL(kb_fb, dim3(L.rest.nblocks), dim3(kWave), 0, s, B, L.rest, n);
   return hipGetLastError();
 }
 

@@ -57,21 +57,19 @@ struct BatchGroup {
   const int32_t* dom;
   const int32_t* prefix;
   int32_t ndom, nblocks, key;
+  int32_t pairs;  // most field pairs of a domain (remap groups)
 };
 constexpr int kMaxGroups = 8;
 struct BatchLaunch {
   int32_t kmax;        // largest kdm of the batch (LDS size)
-  int32_t remap_cols;  // columns per remap workgroup: 64, 128 or 256
   int32_t regrid_cols; // columns per regrid workgroup: 64, 128 or 256
-  int32_t remap_stage; // interface levels a remap lane stages in LDS (0: all)
   BatchGroup regrid;                 // row blocks of regrid_cols, all domains
-  BatchGroup remap[kMaxGroups];      // row blocks of remap_cols, by hybmap + 4*precision
+  BatchGroup remap[kMaxGroups];      // 64-wide row blocks, by hybmap + 4*precision
   int32_t nremap;
-  BatchGroup rows64;                 // 64-wide row blocks, all domains
-  BatchGroup halo_j, halo_i;         // kk x 256-wide slices
+  BatchGroup halo;                   // kk x 256-wide slices of the halo points
   BatchGroup uv[kMaxGroups];         // u+v 64-wide blocks, by uv method + 4*precision
   int32_t nuv;
-  BatchGroup uvall;                  // u+v 64-wide blocks, all domains
+  BatchGroup rest;                   // p+u+v 64-wide blocks, all domains
 };
 // Enqueues one hybgen(m,n,.false.) step of every domain of the batch.
 hipError_t launch_batch(const BatchDevice& B, const BatchLaunch& L, int n, hipStream_t s);

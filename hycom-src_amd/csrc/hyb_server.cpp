@@ -397,7 +397,6 @@ int launch_iteration(hyb_server* s) {
     hw[q] = d.W;
   }
   BatchLaunch L{};
-  L.remap_cols = s->cfg.remap_cols;
   L.regrid_cols = s->cfg.regrid_cols;
   std::vector<int32_t> I;
   batch_layout(hp, na, L, I);

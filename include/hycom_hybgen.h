@@ -302,8 +302,9 @@ typedef struct hyb_domain {
 /* One hybgen(m,n,.false.) step of each of ndom independent domains, of any
  * shapes and kdm (<= 64), FP64 or mixed per domain, enqueued on `stream`.
  * Every phase is one launch over all domains (one per remapper and
- * precision for the remaps), captured once into a HIP graph per batch and
- * replayed; the same domain set on the next call replays the same graph.
+ * precision for the remaps).  The launches' descriptors are prepared once per
+ * domain set and kept for the last four sets of each GPU; preparing a set
+ * does not wait for batches that run.
  * Each domain's result is bitwise the one of hycom_hybgen_device on that
  * domain alone.  Requires nhybrd == kdm and no itracr diagnostics
  * (HYB_EUNSUPPORTED otherwise); HYBGEN_DENFIX, FP64 and mixed domains may
@@ -311,23 +312,19 @@ typedef struct hyb_domain {
 int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream);
 
 /* Online autotuning of the batch kernels' launch shape: while enabled (the
- * default), the first calls of a new domain set each try one candidate,
- * timed with HIP events, and the fastest is kept for that set.  First the
- * remap workgroups: columns per workgroup (64, 128, 256) times the LDS
- * split, the interface levels each column stages in LDS (all kmax-1, or
- * 24 or 12 with the deeper levels read from p as the walk reaches them;
- * at most 64 KB per workgroup); then the regrid's columns per workgroup
- * (256, 128, 64) with the best remap shape.  Results do not depend on the
- * shape. */
+ * default), the first calls of a new domain set each try one candidate for
+ * the regrid's columns per workgroup (256, 128, 64), timed with HIP events,
+ * and the fastest is kept for that set.  The remap runs 64 columns a workgroup
+ * by one wave per pair of fields and stages every interface level.  Results do
+ * not depend on the shape. */
 int hycom_hybgen_batch_autotune(int enable);
 
 /* Widths in use for the last batch: columns per workgroup of the remap
  * and of the regrid; *tuned is 1 once the search has finished. */
 int hycom_hybgen_batch_config(int32_t* remap_cols, int32_t* regrid_cols, int32_t* tuned);
 
-/* The LDS split in use for the last batch: interface levels per column
- * staged in LDS by the remap (*levels) and the batch's largest kdm (*kmax;
- * kmax-1 levels = all staged). */
+/* Interface levels per column staged in LDS by the remap of the last batch
+ * (*levels, kmax-1) and the batch's largest kdm (*kmax). */
 int hycom_hybgen_batch_staged_levels(int32_t* levels, int32_t* kmax);
 
 /* The autotuner's candidates for the last batch, in search order: remap
@@ -359,7 +356,8 @@ typedef struct hyb_server hyb_server;
 typedef struct hyb_server_config {
   int64_t hbm_budget;   /* device bytes for resident domains; 0: 90% of free */
   int32_t max_active;   /* requests stepped per iteration, 1..256; 0: 64    */
-  int32_t remap_cols;   /* columns per remap workgroup 64|128|256; 0: 64    */
+  int32_t remap_cols;   /* 0, 64, 128 or 256; the remap runs 64 columns a
+                           workgroup whichever is given                     */
   int32_t regrid_cols;  /* columns per regrid workgroup 64|128|256; 0: 256  */
   int32_t reserved;
 } hyb_server_config;
