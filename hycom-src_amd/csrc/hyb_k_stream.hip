@@ -168,7 +168,7 @@ hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& 
     }
     if (e != hipSuccess) return e;
     PhaseMark pm(T, s, 5);
-    launch_uv_stream(P, V, W, m, tune, s);
+    launch_uv_stream(P, V, W, m, tune, s, true);
     launch_uv_fallback(P, V, W, m, s);
   }
   return hipGetLastError();

@@ -14,7 +14,7 @@ namespace hyb {
 // layer ahead and waited for in one place (PoRecompute).  One slot per array
 // (PD = 1) beats two (133 VGPRs, 3 waves): 2250x1649x41 call 10.4 against
 // 11.0 ms, 1500x1000x41 WENO 4.03 against 4.29 ms; before, 10.8 and 4.2 ms.
-template <int METHOD, int PD, bool MIXED = false, bool RECOMP = false>
+template <int METHOD, int PD, bool MIXED = false, bool RECOMP = false, bool STAGED = false>
 __global__ void __launch_bounds__(kWave) k_uv_s(KParams P, View V, Scratch W, int nl) {
   extern __shared__ double lds[];
   int j = blockIdx.y + 1;
@@ -25,16 +25,27 @@ __global__ void __launch_bounds__(kWave) k_uv_s(KParams P, View V, Scratch W, in
   const int32_t* msk = isv ? V.iv : V.iu;
   if (msk[c0] == 0) return;
   LaneRow dcol{lds + threadIdx.x, kWave};
-  const bool ok = uv_stream<METHOD, PD, MIXED, RECOMP>(P, V, i, j, nl, isv, dcol);
+  const bool ok =
+      uv_stream<METHOD, PD, MIXED, RECOMP, STAGED>(P, V, i, j, nl, isv, dcol, W.ras);
   W.uvf[c0 + (isv ? V.NIJ : 0)] = ok ? 0 : 1;
 }
 
 template <int M, bool RECOMP>
 static void uv_stream_m(const KParams& P, const View& V, const Scratch& W, int nl, int pd,
-                        hipStream_t s) {
+                        bool staged, hipStream_t s) {
   dim3 w1(kWave);
   dim3 gw3((P.ii + kAlignPad + kWave - 1) / kWave, P.jj, 2);
   const size_t lds = RECOMP ? 0 : sizeof(double) * P.kk * kWave;
+  if constexpr (RECOMP) {
+    // level m of a Robert-Asselin step, whose new bottom is not the old one:
+    // the points whose outputs cannot go in place take the workspace (600x400
+    // x41 tile, 16 % of the points: 668 us, against 280 us and 452 us more for
+    // those points column by column)
+    if (staged && W.ras && P.precision == 0 && pd == 4) {
+      hipLaunchKernelGGL((k_uv_s<M, 1, false, true, true>), gw3, w1, lds, s, P, V, W, nl);
+      return;
+    }
+  }
   if (P.precision == 1)
     hipLaunchKernelGGL((k_uv_s<M, 1, true, RECOMP>), gw3, w1, lds, s, P, V, W, nl);
   else if (pd == 4)
@@ -46,17 +57,17 @@ static void uv_stream_m(const KParams& P, const View& V, const Scratch& W, int n
 }
 
 void launch_uv_stream(const KParams& P, const View& V, const Scratch& W, int nl,
-                      const StreamTuning& tune, hipStream_t s) {
+                      const StreamTuning& tune, hipStream_t s, bool staged) {
   const int m = uv_method(P);
   const int pd = tune.uv_prefetch;
   if (tune.uv_recompute) {
-    if (m == 0) uv_stream_m<0, true>(P, V, W, nl, pd, s);
-    else if (m == 1) uv_stream_m<1, true>(P, V, W, nl, pd, s);
-    else uv_stream_m<3, true>(P, V, W, nl, pd, s);
+    if (m == 0) uv_stream_m<0, true>(P, V, W, nl, pd, staged, s);
+    else if (m == 1) uv_stream_m<1, true>(P, V, W, nl, pd, staged, s);
+    else uv_stream_m<3, true>(P, V, W, nl, pd, staged, s);
   } else {
-    if (m == 0) uv_stream_m<0, false>(P, V, W, nl, pd, s);
-    else if (m == 1) uv_stream_m<1, false>(P, V, W, nl, pd, s);
-    else uv_stream_m<3, false>(P, V, W, nl, pd, s);
+    if (m == 0) uv_stream_m<0, false>(P, V, W, nl, pd, staged, s);
+    else if (m == 1) uv_stream_m<1, false>(P, V, W, nl, pd, staged, s);
+    else uv_stream_m<3, false>(P, V, W, nl, pd, staged, s);
   }
 }
 

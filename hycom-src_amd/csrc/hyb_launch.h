@@ -30,9 +30,10 @@ struct PhaseMark {
 };
 
 // hyb_k_uv.hip: the streaming u/v kernels of time level nl (the points they
-// flag are left to launch_uv_fallback or launch_fallbacks)
+// flag are left to launch_uv_fallback or launch_fallbacks); staged: points
+// whose outputs cannot go in place take W.ras, free by then
 void launch_uv_stream(const KParams& P, const View& V, const Scratch& W, int nl,
-                      const StreamTuning& tune, hipStream_t s);
+                      const StreamTuning& tune, hipStream_t s, bool staged = false);
 // hyb_k_misc.hip
 hipError_t launch_halo(const KParams& P, const View& V, hipStream_t s);
 void launch_diag_pre(const KParams& P, const View& V, int n, hipStream_t s);

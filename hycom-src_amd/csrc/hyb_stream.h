@@ -1019,7 +1019,7 @@ struct FieldSink {  // T, S, tracers; th3d from T and S (hybgen.F90:1549-1569)
     }
   }
 };
-template <class PO>
+template <class PO, bool STAGED = false>
 struct UvSink {  // u or v with the thin-layer rule (hybgen.F90:1858-1865)
   double* uu;
   int64_t S;
@@ -1034,14 +1034,22 @@ struct UvSink {  // u or v with the thin-layer rule (hybgen.F90:1858-1865)
   // two layers above their index (the in-place test of uv_stream), and the
   // old interfaces are summed PD+3 layers ahead of the walk.
   double* dpn = nullptr;
+  // STAGED: a point whose outputs cannot go in place (out != 0) writes them
+  // to the workspace, `out` words from their place in uu, and no dpu; once
+  // the walk has read the column, uv_stream brings them over and forms the new
+  // dpu from p once more.
+  int64_t out = 0;
   HYB_HD void emit(int kc, int64_t at, const double* v, bool certain, bool thick) {
+    const int64_t to = STAGED ? at + out : at;
     if (thick || po->prv <= ptop - kOnemm) {
-      uu[at] = v[0];
+      uu[to] = v[0];
       if (!certain) fix |= 1ull << (kc - 1);
     } else {
-      uu[at] = -ub;
+      uu[to] = -ub;
     }
-    if constexpr (is_recompute<PO>::value) dpn[at] = po->dl;
+    if constexpr (is_recompute<PO>::value) {
+      if (!STAGED || out == 0) dpn[at] = po->dl;
+    }
   }
   // outputs kc..KN all take v (clamped), by the rule of emit.  The levels
   // of p are loaded eight at a time (po stands at level kc).
@@ -1079,10 +1087,11 @@ struct UvSink {  // u or v with the thin-layer rule (hybgen.F90:1858-1865)
     while (fix) {
       const int k = __builtin_ctzll(fix) + 1;
       fix &= fix - 1;
-      double x = uu[(int64_t)(k - 1) * S + c0];
+      const int64_t to = (int64_t)(k - 1) * S + (STAGED ? c0 + out : c0);
+      double x = uu[to];
       x = (x < lo[0]) ? smin[0] : x;
       x = (x > hi[0]) ? smax[0] : x;
-      uu[(int64_t)(k - 1) * S + c0] = x;
+      uu[to] = x;
     }
   }
 };
@@ -2368,12 +2377,16 @@ HYB_HDI void remap_stream(const KParams& P, const View& V, const Scratch& W, int
 // ones as running sums of the new dpu (1806-1810), and the remap of u or v
 // with the thin-layer rule (hybgenbj, 1758-1907).  dcol is the lane's LDS
 // column for the new thicknesses.  Where an output of the in-place walk
-// would overwrite a level not yet read (the test of regrid_stream), it
-// writes pu only and returns false; point_c then redoes the point.
+// would overwrite a level not yet read (ra_pre's test, so an output that ends
+// in the deepest layer counts as safe: without that a point in a few hundred
+// failed, those whose bottom layers are massless and whose new bottom lies a
+// rounding above the old one), it writes pu only and returns false, and
+// point_c redoes the point; with `ras` (STAGED) the point goes through that
+// workspace instead, u in its first K levels and v in its next K.
 // ---------------------------------------------------------------------
-template <int METHOD, int PD, bool MIXED = false, bool RECOMP = false>
+template <int METHOD, int PD, bool MIXED = false, bool RECOMP = false, bool STAGED = false>
 HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bool isv,
-                      const LaneRow& dcol) {
+                      const LaneRow& dcol, double* ras = nullptr) {
   const int K = P.kk;
   const int64_t c0 = ij_of(V, i, j);
   const int64_t S = V.NIJ;
@@ -2388,6 +2401,7 @@ HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bo
   double pr = 0.0;  // prsf(k+1)
   pu[0] = 0.0;
   double q0 = 0.0, q1 = 0.0, q2 = 0.0;  // pres(k-2), pres(k-1), pres(k)
+  double zlast = 0.0;  // the deepest old interface above the bottom
   bool have = false;
   double cand = 0.0;
   // the walk's fast quotients need the old interfaces in order and both
@@ -2410,6 +2424,7 @@ HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bo
     tame &= (dk >= 0.0);
     tame &= tame_p(q3);
     tame &= tame_p(pr);
+    if (q3 > q2) zlast = q2;
     q0 = q1;
     q1 = q2;
     q2 = q3;
@@ -2447,7 +2462,10 @@ HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bo
     }
   }
   const double zx = q2;
-  if ((have && cand < zx) || !tame) return false;
+  // (the mixed form keeps the tighter test: the points it leaves are redone
+  // in FP64)
+  const bool over = have && (MIXED ? cand < zx : cand <= zlast);
+  if (!tame || (!STAGED && over)) return false;
   double* dpu1 = (isv ? V.dpv : V.dpu) + lev4(V, 1, nl);  // level 1
   double* uu1 = (isv ? V.v : V.u) + lev4(V, 1, nl);
   PiSum pi{dpu1, S};
@@ -2455,9 +2473,22 @@ HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bo
   if (RECOMP) {
     // the neighbour is a fixed distance before the point
     PoRecompute po(V.p, V.p - (isv ? V.NI : 1), S, depthu, K, c0);
-    UvSink<PoRecompute> sink{uu1, S, ub, pr, &po, 0ull, dpu1};
-    walk_core<METHOD, 1, PD, MIXED, false, true, false>(K, zx, pi, po, sink, fp, 1, K, 0ull, S, 0,
-                                                        c0);
+    UvSink<PoRecompute, STAGED> sink{uu1, S, ub, pr, &po, 0ull, dpu1};
+    if (STAGED && over)
+      sink.out = ((intptr_t)(ras + (isv ? (int64_t)K * S : 0)) - (intptr_t)uu1) / 8;
+    // (staged outputs may all be out above the old bottom: KO = K)
+    walk_core<METHOD, 1, PD, MIXED, false, true, false>(K, zx, pi, po, sink, fp, 1, K, 0ull, S,
+                                                        STAGED ? K : 0, c0);
+    if (STAGED && over) {
+      stage_column(uu1 + c0, 0, uu1 + c0 + sink.out, S, K, S);
+      double bt = dmin(depthu, 0.5 * (p0[0] + p1[0]));
+#pragma unroll 4
+      for (int k = 1; k <= K; k++) {
+        const double a = dmin(depthu, 0.5 * (p0[(int64_t)k * S] + p1[(int64_t)k * S]));
+        dpu[(int64_t)(k - 1) * S] = dmax(0.0, a - bt);
+        bt = a;
+      }
+    }
   } else {
     PoSum po{dcol};
     UvSink<PoSum> sink{uu1, S, ub, pr, &po};
