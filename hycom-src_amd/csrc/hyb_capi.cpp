@@ -698,7 +698,7 @@ int plan_build(BatchPlan& b, int dev, std::vector<unsigned char>& key, std::vect
   b.hP.swap(hP);
   b.hV.swap(hV);
   b.hW.swap(hW);
-  b.cands = {256, 128, 64};
+  b.cands = {64, 128, 256};
   b.ms.assign(b.cands.size(), -1.0f);
   b.cand = 0;
   b.rep = 0;

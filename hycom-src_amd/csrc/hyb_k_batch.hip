@@ -89,13 +89,14 @@ __device__ __forceinline__ RowPos row_pos(const BatchDevice& B, const BatchGroup
 template <int BW>
 __global__ void __launch_bounds__(BW) __attribute__((amdgpu_waves_per_eu(3)))
 kb_regrid(BatchDevice B, BatchGroup G, int n) {
+  __shared__ double hist[kHist * BW];
   const RowPos r = row_pos(B, G, BW, blockIdx.x);
   const KParams& P = B.P[r.d];
   const View V = gview(B.V, r.d);
   const int i = r.i0 + threadIdx.x;
   if (i < 1 || i > P.ii) return;
   if (V.ip[ij_of(V, i, r.j)] == 0) return;
-  regrid_stream<1>(P, V, gscratch(B.W, r.d), i, r.j, n);
+  regrid_stream<1, true>(P, V, gscratch(B.W, r.d), i, r.j, n, LaneRow{hist + threadIdx.x, BW});
 }
 
 // The p-column remap: 64 columns by one wave per pair of fields (blockDim.y

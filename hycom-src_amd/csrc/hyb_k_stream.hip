@@ -45,15 +45,24 @@ __global__ void __launch_bounds__(kBlock) k_regrid_s(KParams P, View V, Scratch 
   regrid_stream(P, V, W, i, j, n);
 }
 
-// the regrid with its window loaded one iteration ahead, held to 3 waves
-// per SIMD
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
+// The regrid with its window loaded one iteration ahead, held to 3 waves per
+// SIMD (168 VGPRs, 4 spilled).  Bound by the latency of its chain of compares,
+// quotients and branches per level, at 3 waves a SIMD.  A wave a block, so
+// that a row's last block is at most a wave too long and a block's registers
+// come free with its own columns; the interfaces behind the window, which the
+// in-place check looks back at, are kept in LDS (read from pres again, that
+// load was the newest of every level and the level waited for all of them),
+// and what the overturn leaves is carried in registers.  600x400x41 183 ->
+// 107 us, 2250x1649x41 1.55 -> 1.38 ms, 150x100x32 75 -> 68 us.  Two
+// iterations ahead (9 spilled): 108 us, 1.39 ms, 69 us.
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
 k_regrid_a(KParams P, View V, Scratch W, int n) {
+  __shared__ double hist[kHist * kWave];
   int j = blockIdx.y + 1;
-  int i = i_aligned0(V, j) + blockIdx.x * blockDim.x + threadIdx.x;
+  int i = i_aligned0(V, j) + blockIdx.x * kWave + threadIdx.x;
   if (i < 1 || i > P.ii) return;
   if (V.ip[ij_of(V, i, j)] == 0) return;
-  regrid_stream<1>(P, V, W, i, j, n);
+  regrid_stream<1, true>(P, V, W, i, j, n, LaneRow{hist + threadIdx.x, kWave});
 }
 
 // first pass of the Robert-Asselin branch
@@ -102,7 +111,8 @@ hipError_t launch_hybgen_stream(const KParams& P, const View& V, const Scratch& 
     {
       PhaseMark pk(T, s, 6);
       if (tune.regrid_ahead)
-        hipLaunchKernelGGL(k_regrid_a, g2, blk, 0, s, P, V, W, n);
+        hipLaunchKernelGGL(k_regrid_a, dim3((P.ii + kAlignPad + kWave - 1) / kWave, P.jj),
+                           dim3(kWave), 0, s, P, V, W, n);
       else
         hipLaunchKernelGGL(k_regrid_s, g2, blk, 0, s, P, V, W, n);
     }

@@ -40,6 +40,7 @@ namespace hyb {
 constexpr int32_t kUnsafe = 1 << 16;  // kp word: remap this column in remap_fallback
 constexpr int kNFMax = 6;             // fields per remap walk
 constexpr int kKMax = 64;             // largest kdm
+constexpr int kHist = 8;              // interfaces regrid_stream keeps behind its window
 
 // minimum thickness of level k (hybgen.F90:456-466) from the initial
 // interface pk = p(k) and dp0cum(k), qdep == 1; *qh = qhrlx(k+1).
@@ -76,15 +77,28 @@ HYB_HD void shl(double (&a)[W], double v) {
   a[W - 1] = v;
 }
 
+// x, a value just loaded, waited for here: used where a load is rare and
+// sits in a branch, so that the wait stays in the branch too.  (Left to its
+// use after the branches join, the wait is for every outstanding load and is
+// paid whether the branch was taken or not.)
+HYB_HD double arrived(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(x));
+#endif
+  return x;
+}
+
 // ---------------------------------------------------------------------
 // regrid of one p-column (hybgenaj up to the remap)
 // ---------------------------------------------------------------------
 // AHEAD: the pass-3 window's next levels (pres, th3d, theta) are loaded
 // AHEAD (0, 1 or 2) layer iterations before the slide takes them in (more
-// registers)
-template <int AHEAD = 0>
+// registers).  hist: the lane's kHist words (in LDS) for the interfaces that
+// have left the window, which the in-place check looks back at; without it
+// they are read from pres again.
+template <int AHEAD = 0, bool HIST = false>
 HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, int i, int j,
-                           int n) {
+                           int n, LaneRow hist = LaneRow{nullptr, 0}) {
   const int K = P.kk;
   const int64_t c0 = ij_of(V, i, j);
   const int64_t S = V.NIJ;
@@ -101,9 +115,11 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
   const double cusha = qqmn * qqmn * (qqmx - 1.0) / ((qqmx - qqmn) * (qqmx - qqmn));
   const double cushb = 1.0 / qqmn;
   auto cushn = [&](double delp, double dp0) -> double {
-    double qq = dmax(qqmn, dmin(qqmx, delp / dp0));
+    // delp/(dp0*qqmx) is half of delp/dp0, exactly (qqmx = 2)
+    const double r = delp / dp0;
+    double qq = dmax(qqmn, dmin(qqmx, r));
     double a = 1.0 - cushb * qq;
-    return dp0 * (1.0 + cusha * (a * a)) * dmax(1.0, delp / (dp0 * qqmx));
+    return dp0 * (1.0 + cusha * (a * a)) * dmax(1.0, 0.5 * r);
   };
   const double dpthin = kDpthin;
   const double rthin = P.hybthn;
@@ -277,13 +293,16 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
                    P.dp0cum[x - 2], &qh);
     return qh;
   };
+  // p(kp-1..kp+1), theta and th3d of layers kp-1 and kp, kept up to date by
+  // the two steps below (read from memory again, they would cost every wave
+  // another wait)
+  double pkm = pin_a, pkk = pin_b, pkp = pres[(int64_t)kp0 * S];
+  double thkm = FK(theta, kp0 - 1), thk = FK(theta, kp0);
+  double tkm = FK(th3d, kp0 - 1), tk = FK(th3d, kp0);
   {
     const int k = kp;
     const int ka = (k - 2 > 1) ? k - 2 : 1;
-    const double pkk = pres[(int64_t)(k - 1) * S], pkm = pres[(int64_t)(k - 2) * S],
-                 pkp = pres[(int64_t)k * S];
-    const double thk = FK(theta, k);
-    const double tk = FK(th3d, k), tkm = FK(th3d, k - 1), tka = FK(th3d, ka);
+    const double tka = FK(th3d, ka);
     if (k > fixlay + 1 && qdep == 1.0 && pkk - pkm >= dpthin && thk - kEpsil > tk &&
         tkm > tk && tka > tk) {
       // 609-686 entrain layer k into k-1
@@ -295,6 +314,12 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
         TRK(t, k - 1) = TRK(t, k - 1) - q * (TRK(t, k - 1) - TRK(t, k));
       pres[(int64_t)(k - 1) * S] = pkp;
       kp = k - 1;
+      tk = FK(th3d, k - 1);
+      tkm = arrived(FK(th3d, k - 2));
+      thk = thkm;
+      thkm = arrived(FK(theta, k - 2));
+      pkk = pkm;  // and p(kp+1) is still pkp
+      pkm = arrived(pres[(int64_t)(k - 3) * S]);
     } else if (k > fixlay + 1 && qdep == 1.0 && pkk - pkm >= dpthin && thk - kEpsil > tk &&
                tkm > tk) {
       // 687-811 swap with the layer above
@@ -307,6 +332,8 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
         FK(temp, k) = st;
         FK(saln, k) = ss;
         FK(th3d, k) = sh;
+        tk = sh;
+        tkm = FK(th3d, k - 1);
         for (int t = 1; t <= ntracr; t++) {
           double sv = TRK(t, k - 1);
           TRK(t, k - 1) = TRK(t, k - 1) - q * (TRK(t, k - 1) - TRK(t, k));
@@ -321,6 +348,8 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
         FK(temp, k - 1) = st;
         FK(saln, k - 1) = ss;
         FK(th3d, k - 1) = sh;
+        tkm = sh;
+        tk = FK(th3d, k);
         for (int t = 1; t <= ntracr; t++) {
           double sv = TRK(t, k);
           TRK(t, k) = TRK(t, k) + q * (TRK(t, k - 1) - TRK(t, k));
@@ -332,20 +361,22 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
   {
     // 813-970 unmix a too-light deepest layer
     const int k = kp;
-    const double pkk = pres[(int64_t)(k - 1) * S], pkm = pres[(int64_t)(k - 2) * S],
-                 pkp = pres[(int64_t)k * S];
     const double dpthck = P.dx0k[k - 2] * 0.95;
-    const double thk = FK(theta, k), thkm = FK(theta, k - 1);
-    const double tk = FK(th3d, k), tkm = FK(th3d, k - 1);
     if (k > fixlay + 1 && qdep == 1.0 && pkk - pkm >= dpthin && pkk - pkm < dpthck &&
         thk - kEpsil > tk && thkm < tk && dabs(thkm - tkm) < P.hybiso &&
         (tk - tkm) > (thk - thkm) * 0.001) {
+      // the deepest kt <= k-2 that is light enough, eight levels loaded at a
+      // time (clamped to level 2; a clamped one is not looked at)
       int ka = 1;
-      for (int kt = k - 2; kt >= 2; kt--) {
-        if (tkm - FK(th3d, kt) >= thkm - FK(theta, k - 2)) {
-          ka = kt;
-          break;
-        }
+      const double gap = thkm - FK(theta, k - 2);
+      for (int k0 = k - 2; k0 >= 2; k0 -= 8) {
+        double t[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) t[q] = FK(th3d, (k0 - q >= 2) ? k0 - q : 2);
+#pragma unroll
+        for (int q = 7; q >= 0; q--)
+          if (k0 - q >= 2 && tkm - t[q] >= gap) ka = k0 - q;
+        if (ka > 1) break;
       }
       double delsm = dabs(FK(saln, ka) - FK(saln, k - 1));
       double dels = dabs(FK(saln, k - 1) - FK(saln, k));
@@ -373,6 +404,7 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
       FK(temp, k) = FK(temp, k) + (q / (1.0 - q)) * (FK(temp, k) - FK(temp, k - 1));
       FK(saln, k) = FK(saln, k) + (q / (1.0 - q)) * (FK(saln, k) - FK(saln, k - 1));
       FK(th3d, k) = sig(FK(temp, k), FK(saln, k)) - P.thbase;
+      tk = FK(th3d, k);
       if (ntracr > 0 && p_hat != 0.0) {
         double qtr = p_hat / dmax(p_hat, pknew - pkm);
         for (int t = 1; t <= ntracr; t++) {
@@ -387,8 +419,11 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
   }
   // 972-1009 (nhybrd == kk): levels below kp take level kp's values; the
   // remap applies this fill to T, S and the tracers as it loads them.
-  const double th_kp = FK(th3d, kp);
-  auto th3d_eff = [&](int x) -> double { return x > kp ? th_kp : FK(th3d, x); };
+  const double th_kp = tk;
+  auto th3d_eff = [&](int x) -> double {
+    const double t = FK(th3d, x);
+    return x > kp ? th_kp : t;
+  };
 
   // ------------------------------------------------ pass 3: 1036-1529
   const double floor1 = 0.0 + dp0ij1;              // 1053-1055: p(1)+dp0ij(1)
@@ -515,11 +550,20 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
       nta3[q] = theta[clk(5 + q)];
     }
   }
+  // level x as the overturn left it, for x >= 1 above the window (0 before
+  // any use: consume() looks at it from output 4 on, that is from x = 2 on)
+  auto back = [&](int x) -> double { return hist((x & (kHist - 1)) + 1); };
+  if (HIST) {
+#pragma unroll
+    for (int x = 0; x < kHist; x++) hist(x + 1) = 0.0;
+    hist(1 + 1) = raw_at(1);
+    hist(2 + 1) = raw_at(2);
+  }
   double q, p_hat, p_hat0 = 0.0, p_hat2, p_hat3;
 #pragma unroll 1
   for (int k = 2; k <= K; k++) {
     // pres(k-5) for the in-place check of consume(k-2), issued early
-    const double pchk = (k >= 7) ? pres[(int64_t)(k - 6) * S] : 0.0;
+    const double pchk = HIST ? back(k - 5) : (k >= 7) ? pres[(int64_t)(k - 6) * S] : 0.0;
 #define PW(x) pw[(x) - (k - 3)]
     const double dm1 = dw[2], dm2 = dw[1], dm3 = dw[0], d0 = dw[3], dp1 = dw[4];
     const double qm1 = qw[1], qm2 = qw[0], q0 = qw[2], qp1 = qw[3];
@@ -745,12 +789,19 @@ HYB_HDI void regrid_stream(const KParams& P, const View& V, const Scratch& W, in
       qh_next = qh;
       shl(dw, dn);
     }
+    if (HIST) hist(((k + 1) & (kHist - 1)) + 1) = rw[0];
     shl(rw, r4);
   }
   // levels kk-1, kk, kk+1 (pw holds p(kk-2..kk+4) now)
-  consume(K - 1, pw[1], K - 1 >= 5 ? pres[(int64_t)(K - 5) * S] : 0.0);
-  consume(K, pw[2], K >= 5 ? pres[(int64_t)(K - 4) * S] : 0.0);
-  consume(K + 1, pw[3], K + 1 >= 5 ? pres[(int64_t)(K - 3) * S] : 0.0);
+  if (HIST) {
+    consume(K - 1, pw[1], back(K - 4));
+    consume(K, pw[2], back(K - 3));
+    consume(K + 1, pw[3], back(K - 2));
+  } else {
+    consume(K - 1, pw[1], K - 1 >= 5 ? pres[(int64_t)(K - 5) * S] : 0.0);
+    consume(K, pw[2], K >= 5 ? pres[(int64_t)(K - 4) * S] : 0.0);
+    consume(K + 1, pw[3], K + 1 >= 5 ? pres[(int64_t)(K - 3) * S] : 0.0);
+  }
   W.kp[c0] = kp | ((unsafe || !tame) ? kUnsafe : 0);
   W.lcm[c0] = lcm;
   if (V.rec_fixlay) {
@@ -818,16 +869,6 @@ HYB_HD double leave_slot(double x) {
 #endif
 }
 
-// x, a value just loaded, waited for here: used where a load is rare and
-// sits in a branch, so that the wait stays in the branch too.  (Left to its
-// use after the branches join, the wait is for every outstanding load and is
-// paid whether the branch was taken or not.)
-HYB_HD double arrived(double x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("" : "+v"(x));
-#endif
-  return x;
-}
 // the same for a look-ahead slot in place (StokesBlend has its own)
 HYB_HD void slot_arrived(double& x) { x = arrived(x); }
 
