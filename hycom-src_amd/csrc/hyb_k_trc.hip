@@ -7,9 +7,15 @@
 
 namespace hyb {
 
-// plmtrc at 3 waves per SIMD: its chain of 4 fields needs about 200 VGPRs,
-// and at 168 the few that spill cost less than a wave fewer per SIMD (13.3
-// against 16.7 ms at GLBb); pcmtrc fits 4 waves
+// A lane's column by kTrcChunk fields (more fields in further blocks), scanned
+// together.  Bound by the issue and latency of the scan's quotients and of the
+// loads one layer ahead.  plmtrc at 3 waves per SIMD: its chain of 4 fields
+// needs about 200 VGPRs, and at 168 the few that spill cost less than a wave
+// fewer.  1500x1000x41, 4 fields: 1012 us with po(k+1) and pi(lf) read where
+// they were needed, at every output, 955 us with both in registers by then.
+// Slower: a wave per two fields 1115 us, per field 1770 us; lanes that reach
+// the bottom waiting for the wave's other lanes to scan to it together 1110
+// us (their rows are then written twice in part).
 template <int METHOD, int CHUNK, int WPE>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WPE))) k_trc(KTrc Q) {
   const int j = blockIdx.y + 1;
@@ -18,7 +24,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WPE)
   if (i < 1 || i > Q.ii) return;
   const int64_t c0 = trc_ij(Q, i, j);
   if (Q.mask[c0] == 0) return;
-  if (!trc_column_m<METHOD, CHUNK>(Q, c0))
+  if (!trc_chunk<METHOD, CHUNK>(Q, c0, blockIdx.z * CHUNK))
     atomicMin(Q.bad, (int32_t)(c0 < INT_MAX ? c0 : INT_MAX - 1));
 }
 
@@ -27,7 +33,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WPE)
 __global__ void k_trc_reset(int32_t* bad) { *bad = INT_MAX; }
 
 hipError_t launch_trc(const KTrc& Q, hipStream_t s) {
-  dim3 g((Q.ii + kAlignPad + kWave - 1) / kWave, Q.jj);
+  dim3 g((Q.ii + kAlignPad + kWave - 1) / kWave, Q.jj, (Q.ks + kTrcChunk - 1) / kTrcChunk);
   hipLaunchKernelGGL(k_trc_reset, dim3(1), dim3(1), 0, s, Q.bad);
   if (Q.method == 0)
     hipLaunchKernelGGL((k_trc<0, kTrcChunk, 4>), g, dim3(kWave), 0, s, Q);

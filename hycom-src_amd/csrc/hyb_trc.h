@@ -170,6 +170,32 @@ struct TrcChain {
   }
 };
 
+// The outputs of a column, in the two remaps below: scan(zt, zb) forms one
+// output's sums from its layers, emit(k) stores output k.  po(k+1) is loaded
+// an output ahead.
+template <class BAD, class SCAN, class EMIT>
+HYB_HDI bool trc_outputs(const KTrc& Q, const double* po, double zx, const BAD& bad,
+                         const SCAN& scan, const EMIT& emit) {
+  const int64_t S = Q.NIJ;
+  const int ko = Q.ko;
+  bool ok = true;
+  double zb = po[0], zn = po[S];
+  for (int k = 1; k <= ko; k++) {
+    const double zt = zb;
+    zb = zn;
+    zn = po[(int64_t)(k < ko ? k + 1 : ko) * S];
+    if (zb - zt < kTrcThin || zt >= zx) {
+      // thin or bottomed: the output above
+    } else if (bad(zt)) {
+      ok = false;
+    } else {
+      scan(zt, zb);
+    }
+    emit(k);
+  }
+  return ok;
+}
+
 // pcmtrc (808-909) of fields f0..f0+NF-1 of column c0, in one scan of the
 // old layers (the reference's loop over ks inside the loop over l).
 // Returns false where the reference stops ('bad lf', 866-869); that
@@ -180,7 +206,6 @@ HYB_HDI bool trc_pcm_fields(const KTrc& Q, int64_t c0, int f0) {
   const int ki = Q.ki, ko = Q.ko;
   const double thin = kTrcThin;
   const double* pi = Q.pi + c0;
-  const double* po = Q.po + c0;
   const double* si[NF];
   double* so[NF];
 #pragma unroll
@@ -189,65 +214,90 @@ HYB_HDI bool trc_pcm_fields(const KTrc& Q, int64_t c0, int f0) {
     so[f] = Q.so + c0 + S * (int64_t)ko * (f0 + f);
   }
   auto PI = [&](int l) -> double { return pi[(int64_t)(l - 1) * S]; };
-  double prev[NF], sok[NF];
+  double prev[NF];
 #pragma unroll
   for (int f = 0; f < NF; f++) prev[f] = si[f][0];  // the reference reads so(0) here
-  const double zx = PI(ki + 1);
   int lf = 1;
-  double zb = po[0];
-  bool ok = true;
-  for (int k = 1; k <= ko; k++) {
-    const double zt = zb;
-    zb = po[(int64_t)k * S];
-    if (zb - zt < thin || zt >= zx) {
-      // thin or bottomed: the output above
-    } else if (PI(lf) > zt) {
-      ok = false;
+  // layer lf's interfaces and words, kept from one output to the next
+  double h1 = PI(1), h2 = PI(2), hv[NF];
 #pragma unroll
-      for (int f = 0; f < NF; f++) prev[f] = NAN;
-    } else {
-      const double dz = zb - zt;
+  for (int f = 0; f < NF; f++) hv[f] = si[f][0];
+  auto bad = [&](double zt) -> bool {
+    if (!(h1 > zt)) return false;
 #pragma unroll
-      for (int f = 0; f < NF; f++) sok[f] = 0.0;
-      // pi(l), pi(l+1) and layer l's words are in registers when
-      // iteration l starts: each iteration loads layer l+1's while it sums
-      // layer l (a break leaves those loads unused)
-      double pl1 = PI(lf), pl2 = PI(lf + 1);
-      double cv[NF];
+    for (int f = 0; f < NF; f++) prev[f] = NAN;
+    return true;
+  };
+  auto scan = [&](double zt, double zb) {
+    const double dz = zb - zt;
+    double sok[NF];
 #pragma unroll
-      for (int f = 0; f < NF; f++) cv[f] = si[f][(int64_t)(lf - 1) * S];
-      for (int l = lf; l <= ki; l++) {
-        const double pl = pl1;
-        if (pl > zb) {
-          lf = l - 1;
-          break;
-        }
-        pl1 = pl2;
-        const bool more = l + 1 <= ki;
-        double nv[NF];
-        pl2 = more ? PI(l + 2) : 0.0;
+    for (int f = 0; f < NF; f++) sok[f] = 0.0;
+    // pi(l), pi(l+1) and layer l's words are in registers when
+    // iteration l starts: each iteration loads layer l+1's while it sums
+    // layer l (a break leaves those loads unused)
+    double pl1 = h1, pl2 = h2;
+    double pb = 0.0;  // pi(l-1), and layer l-1's words
+    double cv[NF], bv[NF];
+    bool early = false;
 #pragma unroll
-        for (int f = 0; f < NF; f++) nv[f] = more ? si[f][(int64_t)l * S] : 0.0;
-        if (pl >= zt && pl1 <= zb) {
-          const double q = dmax(pl1 - pl, thin) / dz;
-#pragma unroll
-          for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * cv[f];
-        } else {
-          const double bot = dmin(pl1, zb), top = dmax(pl, zt);
-          const double q = dmax(bot - top, thin) / dz;
-#pragma unroll
-          for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * cv[f];
-        }
-#pragma unroll
-        for (int f = 0; f < NF; f++) cv[f] = nv[f];
+    for (int f = 0; f < NF; f++) {
+      cv[f] = hv[f];
+      bv[f] = 0.0;
+    }
+    int l = lf;
+    for (; l <= ki; l++) {
+      const double pl = pl1;
+      if (pl > zb) {
+        early = true;
+        break;
       }
+      pl1 = pl2;
+      const bool more = l + 1 <= ki;
+      double nv[NF];
+      pl2 = more ? PI(l + 2) : 0.0;
 #pragma unroll
-      for (int f = 0; f < NF; f++) prev[f] = sok[f];
+      for (int f = 0; f < NF; f++) nv[f] = more ? si[f][(int64_t)l * S] : 0.0;
+      if (pl >= zt && pl1 <= zb) {
+        const double q = dmax(pl1 - pl, thin) / dz;
+#pragma unroll
+        for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * cv[f];
+      } else {
+        const double bot = dmin(pl1, zb), top = dmax(pl, zt);
+        const double q = dmax(bot - top, thin) / dz;
+#pragma unroll
+        for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * cv[f];
+      }
+      pb = pl;
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        bv[f] = cv[f];
+        cv[f] = nv[f];
+      }
+    }
+    if (early) {
+      if (l > lf) {
+        h1 = pb;
+        h2 = pl1;
+#pragma unroll
+        for (int f = 0; f < NF; f++) hv[f] = bv[f];
+      } else {  // only with zt a NaN: bad() saw pi(lf) <= zt, and zb > zt
+        const int x = l > 1 ? l - 1 : 1;
+        h1 = PI(x);
+        h2 = PI(x + 1);
+#pragma unroll
+        for (int f = 0; f < NF; f++) hv[f] = si[f][(int64_t)(x - 1) * S];
+      }
+      lf = l - 1;
     }
 #pragma unroll
+    for (int f = 0; f < NF; f++) prev[f] = sok[f];
+  };
+  auto emit = [&](int k) {
+#pragma unroll
     for (int f = 0; f < NF; f++) so[f][(int64_t)(k - 1) * S] = prev[f];
-  }
-  return ok;
+  };
+  return trc_outputs(Q, Q.po + c0, PI(ki + 1), bad, scan, emit);
 }
 
 // plmtrc (911-1037) of fields f0..f0+NF-1 of column c0, the slopes formed
@@ -264,7 +314,6 @@ HYB_HDI bool trc_plm_fields(const KTrc& Q, int64_t c0, int f0) {
   const int ki = Q.ki, ko = Q.ko;
   const double thin = kTrcThin;
   const double* pi = Q.pi + c0;
-  const double* po = Q.po + c0;
   const double* si[NF];
   double* so[NF];
 #pragma unroll
@@ -274,7 +323,7 @@ HYB_HDI bool trc_plm_fields(const KTrc& Q, int64_t c0, int f0) {
   }
   TrcChain<NF> ch;
   ch.init(si, pi, S, ki);
-  double prev[NF], sok[NF];
+  double prev[NF];
   uint64_t unc[NF];   // outputs written unclamped
   bool punc[NF];      // prev is unclamped
 #pragma unroll
@@ -283,69 +332,69 @@ HYB_HDI bool trc_plm_fields(const KTrc& Q, int64_t c0, int f0) {
     unc[f] = 0ull;
     punc[f] = false;
   }
-  const double zx = pi[(int64_t)ki * S];
   int lf = 1;
-  double zb = po[0];
-  bool ok = true;
-  for (int k = 1; k <= ko; k++) {
-    const double zt = zb;
-    zb = po[(int64_t)k * S];
-    if (zb - zt < thin || zt >= zx) {
-      // thin or bottomed: the output above
-    } else if (pi[(int64_t)(lf - 1) * S] > zt) {
-      ok = false;
+  double plf = ch.pm;  // pi(lf)
+  auto bad = [&](double zt) -> bool {
+    if (!(plf > zt)) return false;
 #pragma unroll
-      for (int f = 0; f < NF; f++) {
-        prev[f] = NAN;
-        punc[f] = false;
-      }
-    } else {
-      const double dz = zb - zt;
-#pragma unroll
-      for (int f = 0; f < NF; f++) sok[f] = 0.0;
-      if (ch.head > lf) ch.start(false);
-      while (ch.head < lf) ch.advance();
-      // layer l = ch.head: pi(l) = ch.pm, pi(l+1) = ch.p0, si(l) = ch.am,
-      // its slope ch.slope()
-      for (int l = lf;; l++) {
-        const double pl = ch.pm;
-        if (pl > zb) {
-          lf = l - 1;
-          break;
-        }
-        const double pl1 = ch.p0;
-        if (pl >= zt && pl1 <= zb) {
-          const double q = dmax(pl1 - pl, thin) / dz;
-#pragma unroll
-          for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * ch.am[f];
-        } else {
-          const double bot = dmin(pl1, zb), top = dmax(pl, zt);
-          const double q = dmax(bot - top, thin) / dz;
-          const double zc = 0.5 * (bot + top);
-          const double qc = (zc - pl) / dmax(pl1 - pl, thin) - 0.5;
-#pragma unroll
-          for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * (ch.am[f] + qc * ch.slope(f));
-        }
-        if (l == ki) break;  // ran to the last layer: lf stays
-        if (pl1 > zb) {      // layer l+1 starts below the output
-          lf = l;
-          break;
-        }
-        ch.advance();
-      }
-#pragma unroll
-      for (int f = 0; f < NF; f++) {
-        const double v = sok[f];
-        prev[f] = v;
-        punc[f] = !(v >= ch.mn[f] && v <= ch.mx[f]);
-      }
+    for (int f = 0; f < NF; f++) {
+      prev[f] = NAN;
+      punc[f] = false;
     }
+    return true;
+  };
+  auto scan = [&](double zt, double zb) {
+    const double dz = zb - zt;
+    double sok[NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) sok[f] = 0.0;
+    if (ch.head > lf) ch.start(false);
+    while (ch.head < lf) ch.advance();
+    // layer l = ch.head: pi(l) = ch.pm, pi(l+1) = ch.p0, si(l) = ch.am,
+    // its slope ch.slope()
+    for (int l = lf;; l++) {
+      const double pl = ch.pm;
+      if (pl > zb) {  // at l = lf, and only with zt a NaN (bad() saw pi(lf) <= zt)
+        lf = l - 1;
+        plf = pi[(int64_t)(lf > 1 ? lf - 1 : 0) * S];
+        break;
+      }
+      const double pl1 = ch.p0;
+      if (pl >= zt && pl1 <= zb) {
+        const double q = dmax(pl1 - pl, thin) / dz;
+#pragma unroll
+        for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * ch.am[f];
+      } else {
+        const double bot = dmin(pl1, zb), top = dmax(pl, zt);
+        const double q = dmax(bot - top, thin) / dz;
+        const double zc = 0.5 * (bot + top);
+        const double qc = (zc - pl) / dmax(pl1 - pl, thin) - 0.5;
+#pragma unroll
+        for (int f = 0; f < NF; f++) sok[f] = sok[f] + q * (ch.am[f] + qc * ch.slope(f));
+      }
+      if (l == ki) break;  // ran to the last layer: lf stays
+      if (pl1 > zb) {      // layer l+1 starts below the output
+        lf = l;
+        plf = pl;
+        break;
+      }
+      ch.advance();
+    }
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      const double v = sok[f];
+      prev[f] = v;
+      punc[f] = !(v >= ch.mn[f] && v <= ch.mx[f]);
+    }
+  };
+  auto emit = [&](int k) {
 #pragma unroll
     for (int f = 0; f < NF; f++) {
       so[f][(int64_t)(k - 1) * S] = prev[f];
       if (punc[f]) unc[f] |= 1ull << (k - 1);
     }
-  }
+  };
+  const bool ok = trc_outputs(Q, Q.po + c0, pi[(int64_t)ki * S], bad, scan, emit);
   bool any = false;
 #pragma unroll
   for (int f = 0; f < NF; f++) any |= unc[f] != 0ull;
@@ -367,26 +416,28 @@ HYB_HDI bool trc_plm_fields(const KTrc& Q, int64_t c0, int f0) {
   return ok;
 }
 
-// the fields of column c0 in chunks of CHUNK, each chunk one scan
+// the fields of column c0 from f0 on, at most CHUNK, in one scan
+template <int METHOD, int CHUNK>
+HYB_HDI bool trc_chunk(const KTrc& Q, int64_t c0, int f0) {
+  const int nf = Q.ks - f0 < CHUNK ? Q.ks - f0 : CHUNK;
+  if constexpr (METHOD == 0) {
+    if (CHUNK >= 4 && nf == 4) return trc_pcm_fields<(CHUNK >= 4 ? 4 : 1)>(Q, c0, f0);
+    if (CHUNK >= 3 && nf == 3) return trc_pcm_fields<(CHUNK >= 3 ? 3 : 1)>(Q, c0, f0);
+    if (CHUNK >= 2 && nf == 2) return trc_pcm_fields<(CHUNK >= 2 ? 2 : 1)>(Q, c0, f0);
+    return trc_pcm_fields<1>(Q, c0, f0);
+  } else {
+    if (CHUNK >= 4 && nf == 4) return trc_plm_fields<(CHUNK >= 4 ? 4 : 1)>(Q, c0, f0);
+    if (CHUNK >= 3 && nf == 3) return trc_plm_fields<(CHUNK >= 3 ? 3 : 1)>(Q, c0, f0);
+    if (CHUNK >= 2 && nf == 2) return trc_plm_fields<(CHUNK >= 2 ? 2 : 1)>(Q, c0, f0);
+    return trc_plm_fields<1>(Q, c0, f0);
+  }
+}
+
+// the fields of column c0 in chunks of CHUNK
 template <int METHOD, int CHUNK>
 HYB_HDI bool trc_column_m(const KTrc& Q, int64_t c0) {
   bool ok = true;
-  for (int f0 = 0; f0 < Q.ks; f0 += CHUNK) {
-    const int nf = Q.ks - f0 < CHUNK ? Q.ks - f0 : CHUNK;
-    bool r;
-    if (METHOD == 0) {
-      if (CHUNK >= 4 && nf == 4) r = trc_pcm_fields<(CHUNK >= 4 ? 4 : 1)>(Q, c0, f0);
-      else if (CHUNK >= 3 && nf == 3) r = trc_pcm_fields<(CHUNK >= 3 ? 3 : 1)>(Q, c0, f0);
-      else if (CHUNK >= 2 && nf == 2) r = trc_pcm_fields<(CHUNK >= 2 ? 2 : 1)>(Q, c0, f0);
-      else r = trc_pcm_fields<1>(Q, c0, f0);
-    } else {
-      if (CHUNK >= 4 && nf == 4) r = trc_plm_fields<(CHUNK >= 4 ? 4 : 1)>(Q, c0, f0);
-      else if (CHUNK >= 3 && nf == 3) r = trc_plm_fields<(CHUNK >= 3 ? 3 : 1)>(Q, c0, f0);
-      else if (CHUNK >= 2 && nf == 2) r = trc_plm_fields<(CHUNK >= 2 ? 2 : 1)>(Q, c0, f0);
-      else r = trc_plm_fields<1>(Q, c0, f0);
-    }
-    ok = r && ok;
-  }
+  for (int f0 = 0; f0 < Q.ks; f0 += CHUNK) ok = trc_chunk<METHOD, CHUNK>(Q, c0, f0) && ok;
   return ok;
 }
 
