@@ -136,11 +136,9 @@ void batch_layout(const KParams* hP, int nd, BatchLaunch& L, std::vector<int32_t
       return (int64_t)P.jj * ((P.ii + kAlignPad + cols - 1) / cols);
     };
   };
-  // u, v (and p) points: `of` times the 64-wide row blocks
-  auto blocks64 = [](int of) {
-    return [of](const KParams& P) {
-      return of * (int64_t)P.jj * ((P.ii + kAlignPad + 63) / 64);
-    };
+  // u and v points: the 64-wide row blocks twice
+  auto uvblocks = [](const KParams& P) {
+    return 2 * (int64_t)P.jj * ((P.ii + kAlignPad + 63) / 64);
   };
   std::vector<int> all(nd);
   for (int d = 0; d < nd; d++) all[d] = d;
@@ -168,9 +166,11 @@ void batch_layout(const KParams* hP, int nd, BatchLaunch& L, std::vector<int32_t
     std::vector<int> ds;
     for (int d = 0; d < nd; d++)
       if (uv_method_of(hP[d]) + 4 * hP[d].precision == key) ds.push_back(d);
-    if (!ds.empty()) group(ds, blocks64(2), key, &L.uv[L.nuv++]);
+    if (!ds.empty()) group(ds, uvblocks, key, &L.uv[L.nuv++]);
   }
-  group(all, blocks64(3), 0, &L.rest);
+  group(all, [](const KParams& P) {
+    return 3 * (int64_t)((P.jj + kFbRows - 1) / kFbRows) * ((P.ii + 63) / 64);
+  }, 0, &L.rest);
 }
 
 void batch_bind(BatchLaunch& L, const int32_t* dI) {

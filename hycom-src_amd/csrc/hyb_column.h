@@ -1106,6 +1106,9 @@ struct Scratch {
                       // (hybgen_raflag only; NULL: such columns go to column_ra)
 };
 
+// rows of points that one wave of the copy-first kernels looks through
+constexpr int kFbRows = 8;
+
 // Row of per-lane storage in LDS (device) or a local array (host).
 struct LaneRow {
   double* base;

@@ -45,22 +45,19 @@ __global__ void __launch_bounds__(kBlock) k_phase_c(KParams P, View V, int nl) {
   point_c<KC>(P, V, i, j, nl, isv);
 }
 
-// the columns and the u- and v-points left over, in one launch (z: p, u, v)
+// the columns and the u- and v-points left over, in one launch (z: p, u, v).
+// There are none or a few of them: a wave looks through kFbRows rows, their
+// words loaded together (2250x1649x41: 23 us, a row
+// a wave 46 us).
 template <int KC>
 __global__ void __launch_bounds__(kWave) k_fb(KParams P, View V, Scratch W, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  int j = blockIdx.y + 1;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
+  const int j0 = blockIdx.y * kFbRows + 1;
   if (i > P.ii) return;
-  const int64_t c0 = ij_of(V, i, j);
-  if (blockIdx.z == 0) {
-    if (V.ip[c0] == 0) return;
-    if (!(W.kp[c0] & kUnsafe)) return;
-    remap_fallback(P, V, W, i, j, n);
-  } else {
-    const bool isv = blockIdx.z == 2;
-    if ((isv ? V.iv : V.iu)[c0] == 0) return;
-    if (W.uvf[c0 + (isv ? V.NIJ : 0)] == 0) return;
-    point_c<KC>(P, V, i, j, n, isv);
+  for (uint32_t left = left_over(P, V, W, i, j0, blockIdx.z); left; left &= left - 1) {
+    const int j = j0 + __builtin_ctz(left);
+    if (blockIdx.z == 0) remap_fallback(P, V, W, i, j, n);
+    else point_c<KC>(P, V, i, j, n, blockIdx.z == 2);
   }
 }
 
@@ -122,7 +119,7 @@ void launch_ra_fallback(const KParams& P, const View& V, const Scratch& W, int m
 }
 
 void launch_fallbacks(const KParams& P, const View& V, const Scratch& W, int n, hipStream_t s) {
-  dim3 g((P.ii + kWave - 1) / kWave, P.jj, 3);
+  dim3 g((P.ii + kWave - 1) / kWave, (P.jj + kFbRows - 1) / kFbRows, 3);
   HYB_KC_DISPATCH(P.kk, hipLaunchKernelGGL(k_fb<KC>, g, dim3(kWave), 0, s, P, V, W, n));
 }
 

@@ -2549,6 +2549,28 @@ HYB_HD int uv_method(const KParams& P) {
   return 3;
 }
 
+// Which of the points (i, j0..j0+kFbRows-1) are left to the copy-first code:
+// bit r for row j0+r; z = 0 p-columns, 1 u-points, 2 v-points.  (The flag of a
+// land point is scratch: read, not used.)
+HYB_HDI uint32_t left_over(const KParams& P, const View& V, const Scratch& W, int i, int j0,
+                           int z) {
+  const int32_t* mask = z == 0 ? V.ip : z == 1 ? V.iu : V.iv;
+  const int32_t* flag = z == 0 ? W.kp : z == 1 ? W.uvf : W.uvf + V.NIJ;
+  const int32_t bits = z == 0 ? kUnsafe : ~0;
+  int32_t a[kFbRows], b[kFbRows];
+#pragma unroll
+  for (int r = 0; r < kFbRows; r++) {
+    const int64_t c0 = ij_of(V, i, j0 + r <= P.jj ? j0 + r : P.jj);
+    a[r] = mask[c0];
+    b[r] = flag[c0];
+  }
+  uint32_t left = 0;
+#pragma unroll
+  for (int r = 0; r < kFbRows; r++)
+    if (j0 + r <= P.jj && a[r] != 0 && (b[r] & bits) != 0) left |= 1u << r;
+  return left;
+}
+
 // ---------------------------------------------------------------------
 // Remap of a column flagged kUnsafe: copies the column first (1013-1034),
 // then the reference-shaped coefs/walk of hyb_column.h.
