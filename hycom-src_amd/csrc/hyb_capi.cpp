@@ -640,6 +640,7 @@ struct BatchPlan {
   hipEvent_t done = nullptr;  // after the last launch of this plan
   hipStream_t last = nullptr; // that launch's stream
   bool launched = false;
+  bool kept = false;  // a captured graph holds it: never changed again
   int64_t used = 0;
   std::vector<KParams> hP;
   std::vector<View> hV;
@@ -730,6 +731,30 @@ int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) return fail(HYB_EDEVICE, "device ordinal %d out of range", dev);
+  hipStream_t s = (hipStream_t)stream;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(s, &cap));
+  std::vector<KParams> hP(ndom);
+  std::vector<View> hV(ndom);
+  std::vector<Scratch> hW(ndom);
+  if (cap != hipStreamCaptureStatusNone) {
+    // before anything that a capture does not allow (an allocation, a scan)
+    bool known = false;
+    std::lock_guard<std::mutex> lk(g_batch_mu);
+    for (const BatchPlan& q : g_plans[dev]) {
+      bool same = q.ndom == ndom && !q.key.empty();
+      for (int d = 0; same && d < ndom; d++) {
+        const KParams K = kparams_of(D[d].P);
+        const View V = view_of(D[d].P, D[d].F);
+        same = !D[d].P->check_finite && !memcmp(&K, &q.hP[d], sizeof K) &&
+               !memcmp(&V, &q.hV[d], sizeof V);
+      }
+      known = known || same;
+    }
+    if (!known)
+      return fail(HYB_EUNSUPPORTED,
+                  "stream capture: step the domain set (without check_finite) once before it");
+  }
   for (int d = 0; d < ndom; d++)
     if (D[d].P->check_finite) {
       const KParams K = kparams_of(D[d].P);
@@ -737,9 +762,6 @@ int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream
       if ((rc = scan_finite(K, V, n, (hipStream_t)stream))) return rc;
     }
   std::lock_guard<std::mutex> lk(g_batch_mu);
-  std::vector<KParams> hP(ndom);
-  std::vector<View> hV(ndom);
-  std::vector<Scratch> hW(ndom);
   std::vector<unsigned char> key;
   key.reserve(ndom * (sizeof(KParams) + sizeof(View) + sizeof(Scratch)));
   auto add = [&](const void* a, size_t bytes) {
@@ -754,21 +776,38 @@ int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream
     add(&hV[d], sizeof(View));
     add(&hW[d], sizeof(Scratch));
   }
-  BatchPlan* slot = &g_plans[dev][0];
+  BatchPlan* slot = nullptr;
+  int kept = 0;
   for (BatchPlan& q : g_plans[dev]) {
+    kept += q.kept;
     if (q.ndom == ndom && q.key == key) {
       slot = &q;
       break;
     }
-    if (q.used < slot->used) slot = &q;  // else the one not used for longest
+    // else the one not used for longest
+    if (!q.kept && (!slot || q.used < slot->used)) slot = &q;
   }
   BatchPlan& b = *slot;
+  const bool ready = b.ndom == ndom && b.key == key;
+  if (cap != hipStreamCaptureStatusNone) {
+    // The caller's graph reads this set's descriptors at every replay, so they
+    // stay as they are from now on.
+    if (!ready)
+      return fail(HYB_EUNSUPPORTED, "stream capture: step the domain set once before it");
+    if (!b.kept && kept >= kPlans - 1)
+      return fail(HYB_EUNSUPPORTED, "stream capture: %d domain sets are captured already", kept);
+    b.kept = b.tuned = true;
+    b.pending = false;
+    b.used = ++g_batch_clock;
+    g_plan = slot;
+    HIPCHK(launch_batch(b.B, b.L, n, s));
+    return 0;
+  }
   b.used = ++g_batch_clock;
   g_plan = slot;
-  if (b.ndom != ndom || b.key != key) {
+  if (!ready) {
     if ((rc = plan_build(b, dev, key, hP, hV, hW))) return rc;
   }
-  hipStream_t s = (hipStream_t)stream;
   // autotuning: read the pending measurement, move to the next candidate
   if (b.pending) {
     HIPCHK(hipEventSynchronize(b.ev1));

@@ -82,6 +82,7 @@ extern "C" int hostcheck_hybgen(const hyb_params* P, const hyb_fields* F, int m,
 
 static int64_t g_unsafe_cols = 0;
 static int g_uv_recompute = 0;  // 1: the read-ahead regrid, remap and u/v variants
+static int g_as_device = 0;     // 1: the variants the device runs by default
 static int g_split_ns = 7;      // interface levels the split remap stages (the rest from p)
 
 static int64_t g_uv_fallback = 0;
@@ -106,7 +107,10 @@ static void run_stream(const KParams& P, const View& V, int m, int n, int raflag
   for (int j = 1; j <= jj; j++)
     for (int i = 1; i <= ii; i++)
       if (V.ip[ij_of(V, i, j)]) {
-        if (g_uv_recompute) regrid_stream<1>(P, V, W, i, j, n);
+        if (g_as_device) {
+          double hist[kHist];
+          regrid_stream<1, true>(P, V, W, i, j, n, LaneRow{hist, 1});
+        } else if (g_uv_recompute) regrid_stream<1>(P, V, W, i, j, n);
         else regrid_stream(P, V, W, i, j, n);
       }
   int64_t unsafe = 0;
@@ -129,6 +133,19 @@ static void run_stream(const KParams& P, const View& V, int m, int n, int raflag
           case 1: remap_mixed<1, 3, 2>(P, V, W, i, j, n, po); break;
           case 2: remap_mixed<2, 3, 2>(P, V, W, i, j, n, po); break;
           default: remap_mixed<3, 3, 2>(P, V, W, i, j, n, po); break;
+        }
+        continue;
+      }
+      if (g_as_device) {
+        double srow[kKMax + 2];
+        StagedInterfaces pa = stage_interfaces(srow, 1, V.p + c0, V.NIJ, kk);
+        for (int q = 0; q < field_pairs(P); q++) {
+          switch (P.hybmap) {
+            case 0: remap_pair<0, 2, false>(P, V, W, c0, n, W.kp[c0], q, pa); break;
+            case 1: remap_pair<1, 2, false>(P, V, W, c0, n, W.kp[c0], q, pa); break;
+            case 2: remap_pair<2, 2, false>(P, V, W, c0, n, W.kp[c0], q, pa); break;
+            default: remap_pair<3, 2, false>(P, V, W, c0, n, W.kp[c0], q, pa); break;
+          }
         }
         continue;
       }
@@ -206,6 +223,19 @@ static void run_stream(const KParams& P, const View& V, int m, int n, int raflag
               case 1: ok = uv_stream<1, 4, true, true>(P, V, i, j, nl, isv != 0, dcol); break;
               default: ok = uv_stream<3, 4, true, true>(P, V, i, j, nl, isv != 0, dcol); break;
             }
+          } else if (g_as_device && pass == 1) {
+            const bool v = isv != 0;
+            switch (uv_method(P)) {
+              case 0: ok = uv_stream<0, 1, false, true, true>(P, V, i, j, nl, v, dcol, W.ras); break;
+              case 1: ok = uv_stream<1, 1, false, true, true>(P, V, i, j, nl, v, dcol, W.ras); break;
+              default: ok = uv_stream<3, 1, false, true, true>(P, V, i, j, nl, v, dcol, W.ras); break;
+            }
+          } else if (g_as_device) {
+            switch (uv_method(P)) {
+              case 0: ok = uv_stream<0, 1, false, true>(P, V, i, j, nl, isv != 0, dcol); break;
+              case 1: ok = uv_stream<1, 1, false, true>(P, V, i, j, nl, isv != 0, dcol); break;
+              default: ok = uv_stream<3, 1, false, true>(P, V, i, j, nl, isv != 0, dcol); break;
+            }
           } else if (g_uv_recompute) {
             switch (uv_method(P)) {
               case 0: ok = uv_stream<0, 4, false, true>(P, V, i, j, nl, isv != 0, dcol); break;
@@ -243,6 +273,15 @@ extern "C" int hostcheck_hybgen_stream_rc(const hyb_params* P, const hyb_fields*
   g_uv_recompute = 1;
   const int rc = hostcheck_hybgen_stream(P, F, m, n, raflag);
   g_uv_recompute = 0;
+  return rc;
+}
+
+// the streaming family as the device runs it by default
+extern "C" int hostcheck_hybgen_stream_dev(const hyb_params* P, const hyb_fields* F, int m,
+                                           int n, int raflag) {
+  g_as_device = 1;
+  const int rc = hostcheck_hybgen_stream(P, F, m, n, raflag);
+  g_as_device = 0;
   return rc;
 }
 

@@ -1,0 +1,146 @@
+"""GPU: the branches of the launch rules at the sizes where they turn, against
+the oracle or another path, bitwise.  Every case prints its name first."""
+import numpy as np
+import pytest
+
+import hybgen_abi as abi
+import oracle_lib as ol
+
+pytestmark = pytest.mark.gpu
+
+
+def _host(workload="cfg1", seed=7, extreme=0, **over):
+    P, w = abi.workload_params(workload, **over)
+    return P, abi.HostDomain(P).synth(abi.make_synth(P, w, seed=seed, extreme=extreme))
+
+
+@pytest.mark.parametrize("raflag", [0, 1])
+@pytest.mark.parametrize("ntracr", [0, 1, 5, 6, 7, 11])
+def test_field_pairs(gpu, ntracr, raflag):
+    """One to seven pairs of fields, the last one half empty or not, over one
+    and two blocks of waves, three steps on one state."""
+    import torch
+    print(f"\n[case] field pairs ntracr={ntracr} raflag={raflag}", flush=True)
+    P, d0 = _host(idm=67, jdm=18, kdm=22, ntracr=ntracr, trcflg=[2, 0] * 6 if ntracr else ())
+    want = d0.copy()
+    dd = abi.DeviceDomain(P).upload(d0)
+    for step in range(3):
+        ol.run_oracle(want, m=1, n=2, raflag=raflag, threads=8)
+        dd.hybgen(m=1, n=2, raflag=raflag)
+        torch.cuda.synchronize()
+        df = ol.diff_domains(want, dd.download())
+        assert not df, f"step {step}: {df}"
+
+
+@pytest.mark.parametrize("jdm", [20, 23, 33])
+@pytest.mark.parametrize("hybmap", [2, 3])
+def test_left_over_rows(gpu, jdm, hybmap):
+    """Extreme columns, which the walks leave over, with rows that do and do
+    not fill the last block of eight, on both kernels that look for them."""
+    import torch
+    print(f"\n[case] left-over rows jdm={jdm} hybmap={hybmap}", flush=True)
+    P, d0 = _host(idm=65, jdm=jdm, kdm=32, ntracr=1, trcflg=[0], hybmap=hybmap, extreme=1)
+    want = d0.copy()
+    ol.run_oracle(want, m=1, n=2, threads=8)
+    a = abi.DeviceDomain(P).upload(d0)
+    b = abi.DeviceDomain(P).upload(d0)
+    a.hybgen(m=1, n=2)
+    abi.Batch([b]).hybgen(m=1, n=2)
+    torch.cuda.synchronize()
+    for got in (a, b):
+        assert not ol.diff_domains(want, got.download())
+
+
+# 64-wide tiles x (pairs + 2) of 24576 waves decide between one launch of the
+# remap with the u/v phase and two
+@pytest.mark.parametrize("idm,jdm", [(500, 767), (500, 769)])
+def test_one_launch_line(gpu, idm, jdm):
+    import torch
+    print(f"\n[case] one launch or two, {idm}x{jdm}", flush=True)
+    P, w = abi.workload_params("cfg1", idm=idm, jdm=jdm, kdm=16, ntracr=2, trcflg=[2, 0])
+    S = abi.make_synth(P, w, seed=3)
+    a = abi.DeviceDomain(P).synth(S)
+    b = abi.DeviceDomain(P).synth(S)
+    abi.check(abi.load().hycom_hybgen_tune(4, 1))  # two launches, side by side
+    try:
+        a.hybgen(m=1, n=2)
+    finally:
+        abi.check(abi.load().hycom_hybgen_tune(4, 0))
+    b.hybgen(m=1, n=2)
+    torch.cuda.synchronize()
+    assert not [f for f in abi.OUTPUTS if not torch.equal(a.t[f], b.t[f])]
+
+
+def _sets(count):
+    out = []
+    for q in range(count):
+        P, d0 = _host(idm=40 + 9 * q, jdm=30, kdm=16 + q, seed=q, ntracr=q % 3,
+                      trcflg=[2, 0][:q % 3])
+        out.append((abi.DeviceDomain(P).upload(d0), abi.DeviceDomain(P).upload(d0)))
+    return out
+
+
+def test_more_domain_sets_than_are_kept(gpu):
+    """Six sets in turn, twice the number of steps each, against single calls."""
+    import torch
+    print("\n[case] six domain sets in turn", flush=True)
+    doms = _sets(6)
+    batches = [abi.Batch([doms[q][0], doms[(q + 1) % 6][0]]) for q in range(6)]
+    for _ in range(2):
+        for q, b in enumerate(batches):
+            b.hybgen(m=1, n=2)
+            doms[q][1].hybgen(m=1, n=2)
+            doms[(q + 1) % 6][1].hybgen(m=1, n=2)
+    torch.cuda.synchronize()
+    for a, b in doms:
+        assert not [f for f in abi.OUTPUTS if not torch.equal(a.t[f], b.t[f])]
+
+
+def test_batch_in_a_captured_graph(gpu):
+    """A captured set's descriptors outlive other sets; a set that has not
+    been stepped before is refused."""
+    import torch
+    print("\n[case] batch under stream capture", flush=True)
+    doms = _sets(6)
+    batch = abi.Batch([doms[0][0], doms[1][0]])
+    s = torch.cuda.Stream()
+    fresh = abi.Batch([doms[5][0]])
+    batch.hybgen(m=1, n=2, stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    refused = None
+    with torch.cuda.graph(g, stream=s, capture_error_mode="thread_local"):
+        at = torch.cuda.current_stream().cuda_stream
+        batch.hybgen(m=1, n=2, stream=at)
+        try:
+            fresh.hybgen(m=1, n=2, stream=at)
+        except abi.HybError as e:
+            refused = e
+    assert refused is not None
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        for q in range(2, 6):  # four more sets: as many as are kept
+            abi.Batch([doms[q][0]]).hybgen(m=1, n=2)
+            doms[q][1].hybgen(m=1, n=2)
+        torch.cuda.synchronize()
+    batch.hybgen(m=1, n=2)
+    for _ in range(5):  # one call, three replays, one call
+        doms[0][1].hybgen(m=1, n=2)
+        doms[1][1].hybgen(m=1, n=2)
+    torch.cuda.synchronize()
+    for a, b in doms:
+        assert not [f for f in abi.OUTPUTS if not torch.equal(a.t[f], b.t[f])]
+
+
+@pytest.mark.parametrize("method", [0, 1])
+@pytest.mark.parametrize("ki,ko,ks", [(2, 1, 5), (3, 41, 8), (41, 2, 9)])
+def test_trc_chunks_and_edges(gpu, method, ki, ko, ks):
+    import ctypes
+    from test_trc import _fields, _grid
+    print(f"\n[case] trc method={method} ki={ki} ko={ko} ks={ks}", flush=True)
+    P, a = _grid(np.random.default_rng(ki + 7 * ko + method), method, ki, ko, ks)
+    b = {k: v.copy(order="F") for k, v in a.items()}
+    assert ol.oracle().oracle_trc_remap(ctypes.byref(P), ctypes.byref(_fields(a))) == 0
+    abi.check(abi.load().hycom_trc_remap(ctypes.byref(P), ctypes.byref(_fields(b))))
+    assert np.array_equal(a["so"], b["so"])
