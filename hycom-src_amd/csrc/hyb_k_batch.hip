@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(kBlock) kb_halo(BatchDevice B, BatchGroup G) {
   if (t < P.ii + P.jj + 2) p_halo_point(P, gview(B.V, d), t, local / nb + 2);
 }
 
-// u- and v-points: the first half of a domain's blocks are u, then v
+// u- and v-points: u and v of the same columns in turn, as in k_uv_s
 template <int METHOD, bool MIXED>
 __global__ void __launch_bounds__(kWave) kb_uv(BatchDevice B, BatchGroup G, int nl) {
   extern __shared__ double lds[];
@@ -152,8 +152,8 @@ __global__ void __launch_bounds__(kWave) kb_uv(BatchDevice B, BatchGroup G, int 
   const View V = gview(B.V, d);
   const int nbi = (P.ii + kAlignPad + kWave - 1) / kWave;
   int local = blockIdx.x - G.prefix[g];
-  const bool isv = local >= P.jj * nbi;
-  if (isv) local -= P.jj * nbi;
+  const bool isv = local & 1;
+  local >>= 1;
   const int j = local / nbi + 1;
   const int i = i_aligned0(V, j) + (local % nbi) * kWave + threadIdx.x;
   if (i < 1 || i > P.ii) return;

@@ -7,7 +7,9 @@
 
 namespace hyb {
 
-// A wave per 64 u- or v-points.  Bound by the latency of its walk's loads at
+// A wave per 64 u- or v-points, u and v of the same columns next to each other
+// (they share p; all u first, then all v, read it from memory twice:
+// 2250x1649x41 3540 against 3491 us, 1500x1000x41 1675 against 1650 us).  Bound by the latency of its walk's loads at
 // the occupancy its registers allow: with the column's arrays addressed from
 // uniform bases the walk takes 125 VGPRs, 4 waves a SIMD (138 and 3 with a
 // pointer per lane and array), and every word of a layer is asked for one
@@ -18,8 +20,8 @@ template <int METHOD, int PD, bool MIXED = false, bool RECOMP = false, bool STAG
 __global__ void __launch_bounds__(kWave) k_uv_s(KParams P, View V, Scratch W, int nl) {
   extern __shared__ double lds[];
   int j = blockIdx.y + 1;
-  int i = i_aligned0(V, j) + blockIdx.x * blockDim.x + threadIdx.x;
-  bool isv = blockIdx.z != 0;
+  const bool isv = blockIdx.x & 1;
+  int i = i_aligned0(V, j) + (blockIdx.x >> 1) * kWave + threadIdx.x;
   if (i < 1 || i > P.ii) return;
   const int64_t c0 = ij_of(V, i, j);
   const int32_t* msk = isv ? V.iv : V.iu;
@@ -34,7 +36,7 @@ template <int M, bool RECOMP>
 static void uv_stream_m(const KParams& P, const View& V, const Scratch& W, int nl, int pd,
                         bool staged, hipStream_t s) {
   dim3 w1(kWave);
-  dim3 gw3((P.ii + kAlignPad + kWave - 1) / kWave, P.jj, 2);
+  dim3 gw3(2 * ((P.ii + kAlignPad + kWave - 1) / kWave), P.jj);
   const size_t lds = RECOMP ? 0 : sizeof(double) * P.kk * kWave;
   if constexpr (RECOMP) {
     // level m of a Robert-Asselin step, whose new bottom is not the old one:
