@@ -2504,8 +2504,9 @@ HYB_HDI bool uv_stream(const KParams& P, const View& V, int i, int j, int nl, bo
   }
   const double zx = q2;
   // (the mixed form keeps the tighter test: the points it leaves are redone
-  // in FP64)
-  const bool over = have && (MIXED ? cand < zx : cand <= zlast);
+  // in FP64; so does the variant with the thicknesses in LDS, which only a
+  // tuning knob selects and which keeps point_c in use on ordinary fields)
+  const bool over = have && (MIXED || !RECOMP ? cand < zx : cand <= zlast);
   if (!tame || (!STAGED && over)) return false;
   double* dpu1 = (isv ? V.dpv : V.dpu) + lev4(V, 1, nl);  // level 1
   double* uu1 = (isv ? V.v : V.u) + lev4(V, 1, nl);
