@@ -69,7 +69,7 @@ struct BatchLaunch {
   BatchGroup halo;                   // kk x 256-wide slices of the halo points
   BatchGroup uv[kMaxGroups];         // u+v 64-wide blocks, by uv method + 4*precision
   int32_t nuv;
-  BatchGroup rest;                   // p+u+v 64-wide blocks, all domains
+  BatchGroup rest;                   // p+u+v blocks of 64 columns by kFbRows rows, all domains
 };
 // Enqueues one hybgen(m,n,.false.) step of every domain of the batch.
 hipError_t launch_batch(const BatchDevice& B, const BatchLaunch& L, int n, hipStream_t s);

@@ -304,7 +304,10 @@ typedef struct hyb_domain {
  * Every phase is one launch over all domains (one per remapper and
  * precision for the remaps).  The launches' descriptors are prepared once per
  * domain set and kept for the last four sets of each GPU; preparing a set
- * does not wait for batches that run.
+ * does not wait for batches that run.  In a stream capture the launches are
+ * recorded, if the set has been stepped before (without check_finite); its
+ * descriptors are kept from then on, for at most three sets a GPU.  Other
+ * captures are refused with HYB_EUNSUPPORTED.
  * Each domain's result is bitwise the one of hycom_hybgen_device on that
  * domain alone.  Requires nhybrd == kdm and no itracr diagnostics
  * (HYB_EUNSUPPORTED otherwise); HYBGEN_DENFIX, FP64 and mixed domains may
@@ -313,7 +316,7 @@ int hycom_hybgen_batch(const hyb_domain* D, int ndom, int m, int n, void* stream
 
 /* Online autotuning of the batch kernels' launch shape: while enabled (the
  * default), the first calls of a new domain set each try one candidate for
- * the regrid's columns per workgroup (256, 128, 64), timed with HIP events,
+ * the regrid's columns per workgroup (64, 128, 256), timed with HIP events,
  * and the fastest is kept for that set.  The remap runs 64 columns a workgroup
  * by one wave per pair of fields and stages every interface level.  Results do
  * not depend on the shape. */
