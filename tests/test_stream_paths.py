@@ -56,3 +56,19 @@ def test_robert_asselin_points_take_the_workspace():
         ol.run_oracle(want, m=1, n=2, raflag=1, threads=8)
         assert _step(P, d, 1, 2, 1) == 0
         assert not ol.diff_domains(want, d)
+
+
+@pytest.mark.parametrize("kdm,hybmap,zlevel", [(4, 2, 0), (16, 1, 1), (27, 3, 0), (41, 2, 1),
+                                               (64, 0, 0)])
+def test_denfix_search_matches_oracle(kdm, hybmap, zlevel):
+    few = {"nsigma": kdm} if kdm < 16 else {}
+    P, w = abi.workload_params("cfg1", idm=43, jdm=31, kdm=kdm, hybmap=hybmap, ntracr=1,
+                               ldenfix=1, **few)
+    got = abi.HostDomain(P).synth(abi.make_synth(P, w, seed=kdm))
+    if zlevel:
+        ol.zlevel_start(got, seed=kdm)
+    want = got.copy()
+    for step in range(3):
+        ol.run_oracle(want, m=1, n=2, threads=8)
+        _step(P, got, 1, 2, 0)
+        assert not ol.diff_domains(want, got), f"step {step}"
